@@ -49,24 +49,73 @@ __global__ void copy_kernel(const float *__restrict__ s, float *__restrict__ d, 
         d[i] = s[i];
 }
 
-// norm (elementwise.metal:31-46): one wave per head,
+// norm (elementwise.metal:31-46): one block per head,
 // y[head*n + i] = x[head*stride + i] * rsqrt(mean(x^2) + eps) * w[i].
-template <int T>
-__global__ __launch_bounds__(64) void norm_kernel(const float *__restrict__ x, const void *w,
-                                                  float *__restrict__ y, uint32_t n,
-                                                  uint32_t stride, float eps) {
-    const uint32_t head = blockIdx.x;
-    const int lane = threadIdx.x;
+// Latency-bound: a head's row is a few KB, so what counts is how many of its
+// loads are in flight.  Up to 256 threads hold kNormHold groups of four
+// values each; a row that fits them (n <= 2048) is read once, all its loads
+// issued before the sum.  For one row of 2048 values one wave per head with a
+// load per iteration took 17-20 us by the launch's own events, this form 4.0
+// (of which about 2 are the launch; 24 rows: 24 -> 4 us).
+typedef float f32x4e __attribute__((ext_vector_type(4)));
+constexpr uint32_t kNormThreads = 256, kNormHold = 2;
+
+template <int T, bool VEC>
+__global__ __launch_bounds__(kNormThreads) void norm_kernel(const float *__restrict__ x, const void *w,
+                                                            float *__restrict__ y, uint32_t n,
+                                                            uint32_t stride, float eps) {
+    __shared__ float part[kNormThreads / 64];
+    const uint32_t head = blockIdx.x, tid = threadIdx.x, step = 4 * blockDim.x;
     const float *xr = x + (uint64_t)head * stride;
+    float *yr = y + (uint64_t)head * n;
+    // four values from i on (0 past the end); VEC: n, stride and the bases
+    // allow 16-byte accesses
+    auto load4 = [&](uint32_t i) -> f32x4e {
+        f32x4e v = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (VEC) {
+            if (i < n) v = *reinterpret_cast<const f32x4e *>(xr + i);
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++)
+                if (i + j < n) v[j] = xr[i + j];
+        }
+        return v;
+    };
+    f32x4e hold[kNormHold];
     float s = 0.f;
-    for (uint32_t i = lane; i < n; i += 64) {
-        const float v = xr[i];
-        s += v * v;
+#pragma unroll
+    for (uint32_t q = 0; q < kNormHold; q++) hold[q] = load4(4 * tid + q * step);
+#pragma unroll
+    for (uint32_t q = 0; q < kNormHold; q++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) s += hold[q][j] * hold[q][j];
+    for (uint32_t i = 4 * tid + kNormHold * step; i < n; i += step) {
+        const f32x4e v = load4(i);
+#pragma unroll
+        for (int j = 0; j < 4; j++) s += v[j] * v[j];
     }
     s = wave_sum(s);
+    if ((tid & 63) == 0) part[tid >> 6] = s;
+    __syncthreads();
+    s = 0.f;
+    for (uint32_t k = 0; k < blockDim.x / 64; k++) s += part[k];
     const float inv = 1.0f / sqrtf(s / (float)n + eps);
-    for (uint32_t i = lane; i < n; i += 64)
-        y[(uint64_t)head * n + i] = xr[i] * inv * load_scalar<T>(w, i);
+    auto store4 = [&](uint32_t i, f32x4e v) {
+        if constexpr (VEC) {
+            if (i >= n) return;
+            f32x4e o;
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[j] = v[j] * inv * load_scalar<T>(w, i + j);
+            *reinterpret_cast<f32x4e *>(yr + i) = o;
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++)
+                if (i + j < n) yr[i + j] = v[j] * inv * load_scalar<T>(w, i + j);
+        }
+    };
+#pragma unroll
+    for (uint32_t q = 0; q < kNormHold; q++) store4(4 * tid + q * step, hold[q]);
+    for (uint32_t i = 4 * tid + kNormHold * step; i < n; i += step) store4(i, load4(i));
 }
 
 // out[t, i] = sum_k w[t,k] * yexp[pos[t*K+k]*h + i]          (mix, k ascending)
@@ -113,8 +162,15 @@ hipError_t launch_copy(Prof *p, hipStream_t s, const float *src, float *dst, uin
 
 hipError_t launch_norm(Prof *p, hipStream_t s, const float *x, const void *w, uint32_t wtype,
                        float *y, uint32_t heads, uint32_t n, uint32_t stride, float eps) {
-    auto kern = wtype == 0 ? norm_kernel<0> : wtype == 1 ? norm_kernel<1> : norm_kernel<30>;
-    return launch_kernel(p, "norm", kern, dim3(heads), dim3(64), 0, s, x, w, y, n, stride, eps);
+    // 16-byte accesses where every row starts 16-byte aligned
+    const bool vec = n % 4 == 0 && stride % 4 == 0 &&
+                     ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15u) == 0;
+    auto kern = vec ? (wtype == 0 ? norm_kernel<0, true> : wtype == 1 ? norm_kernel<1, true> : norm_kernel<30, true>)
+                    : (wtype == 0 ? norm_kernel<0, false> : wtype == 1 ? norm_kernel<1, false> : norm_kernel<30, false>);
+    // short rows (attention heads) keep one wave: four values a lane
+    const uint32_t groups = (n + 3) / 4;
+    const uint32_t threads = groups < kNormThreads ? (groups + 63) / 64 * 64 : kNormThreads;
+    return launch_kernel(p, "norm", kern, dim3(heads), dim3(threads), 0, s, x, w, y, n, stride, eps);
 }
 
 hipError_t launch_combine(Prof *p, hipStream_t s, const float *yexp, const uint32_t *pos,

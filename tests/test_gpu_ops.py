@@ -326,3 +326,36 @@ def test_allocation_error_carries_bytes(gpu):
     from hip_backend.api import _lib
     assert _lib.moe_last_error_bytes(gpu._h) == 0
     gpu.release(b)
+
+
+@pytest.mark.parametrize("n,heads,pad", [(1, 2, 0), (64, 5, 3), (128, 16, 0), (255, 2, 1), (260, 3, 4), (1023, 1, 0),
+                                         (2047, 2, 0), (2048, 3, 0), (2052, 2, 0), (5000, 2, 8)])
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+def test_norm_rows(gpu, n, heads, pad, dtype):
+    """Batch::norm at the edges of its block: rows shorter than a wave, of
+    whole and ragged groups of four, rows past the values a block holds, padded
+    strides, and an input that is not 16-byte aligned.  F32 sums of n products:
+    n * 2^-24 is far below the 2e-4 the op's fixture uses."""
+    print(f"[case] norm n={n} heads={heads} pad={pad} dtype={dtype}", flush=True)
+    stride = n + pad
+    x = synth.normal(900 + n, 1 + (heads - 1) * stride + n)
+    w = synth.normal(901 + n, n, 1.0, 0.1)
+    if dtype == F32:
+        t, wf = Tensor.dense([n], w), w
+    elif dtype == BF16:
+        bits = synth.f32_to_bf16_bits(w)
+        t, wf = Tensor.dense([n], bits, BF16), synth.bf16_bits_to_f32(bits)
+    else:
+        h = w.astype(np.float16)
+        t, wf = Tensor.dense([n], h.view(np.uint16), F16), h.astype(np.float32)
+    wt, buf = gpu.weight_tensor(t), gpu.upload(x)
+    for first in (0, 1):  # aligned, and one element off
+        y = gpu.zeros(heads * n)
+        with gpu.batch() as b:
+            b.norm(buf.view(first, len(x) - 1), wt, y, heads, stride, 1e-5)
+        got = gpu.read(y).reshape(heads, n)
+        for i in range(heads):
+            row = x[first + i * stride:first + i * stride + n]
+            close(got[i], oracle.rms_norm(row, wf, 1e-5), 2e-4)
+        gpu.release(y)
+    gpu.release(buf)
