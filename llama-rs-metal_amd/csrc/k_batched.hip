@@ -87,12 +87,7 @@ struct InChunk {
             v[4 * i + 3] = q.w;
         }
     }
-    __device__ __forceinline__ float sum() const {
-        float s = 0.f;
-#pragma unroll
-        for (int j = 0; j < 32; j++) s += v[j];
-        return s;
-    }
+    __device__ __forceinline__ float sum() const { return sum32(v); }
 };
 
 // Runs `body(chunk, p)` for p in [beg, end), the chunk of input row row_of(p)
@@ -240,7 +235,7 @@ __global__ __launch_bounds__(64) void seg_rows_kernel(SegArgs a) {
     auto body = [&](const InChunk &X, uint32_t p) {
         L.pin();  // convert the codes per input row: all rows' would not fit
         float res[kSegRowsFR];
-        L.dot(X.v, X.sum(), res);
+        L.template dot<BITS == 4>(X.v, X.sum(), res);
 #pragma unroll
         for (int f = 0; f < kSegRowsFR; f++) {
             const float v = subwave_sum(res[f], (int)lpr);
