@@ -34,7 +34,8 @@ struct DecodeKArgs {
     WDesc router, gate, up, down, sg, su, sd, sgi;
     uint32_t has_shared, k, normalize;
     uint32_t h, ff, ffs, E;
-    uint32_t lpr_h, lpr_f;  // lanes per row along h / along ff (powers of two <= 64)
+    uint32_t lpr_h, lpr_f;  // lanes per row along h / along ff (powers of two <= 64); a row
+                            // of ff spans lpr_f lanes x CPL chunks (decode_down)
     uint32_t n_router_waves, n_shared_waves, n_gate_waves_per_expert;
     const float *x, *norm_w, *logit_bias, *resid;
     float eps;
@@ -43,7 +44,11 @@ struct DecodeKArgs {
     float *weights, *act, *sh_act, *sh_gate;
 };
 
-constexpr int kDownFR = 2;    // output rows per sub-wave in decode_down
+// Output rows per sub-wave in decode_down: two of one chunk per lane, or one
+// of three (ff = 3 * 2^k chunks), so a block covers 8 rows of 512 or of 768
+// values and h 2048 fills the 256 CUs with one block each.
+template <int CPL>
+constexpr int down_rows() { return CPL == 1 ? 2 : 1; }
 constexpr int kPreFR = 2;     // router rows per sub-wave in decode_pre (one input slice each)
 
 // ------------------------------------------------------------------ pre --
@@ -217,14 +222,14 @@ __global__ __launch_bounds__(64) void decode_gateup_kernel(DecodeKArgs a) {
 // w, w+nw, ... of the K routed experts plus the shared one (index K); all of
 // a wave's weight loads are issued before its arithmetic, its expert's
 // activation row reaches every sub-wave through the wave's LDS slot
-// (staged_row), and the waves' partial sums meet in LDS.
+// (stage_row), and the waves' partial sums meet in LDS.
 constexpr int kDownMaxWaves = 16;
 constexpr int kDownMaxPerWave = 2;
 constexpr size_t kDownSlotBytes = 48 * 1024;  // beside the 16 KiB combine arrays
 
-// This wave's activation row (ff floats) into xr: with a slot, through the
-// wave's own LDS slot -- lane l loads float4s l, l + 64, ... once and every
-// sub-wave reads its chunk from LDS (float4 i of chunk c at slot i * C + c,
+// This wave's activation row (ff floats): with a slot, through the wave's own
+// LDS slot -- lane l loads float4s l, l + 64, ... once (stage_row) and every
+// sub-wave reads its chunks from LDS (float4 i of chunk c at slot i * C + c,
 // so a sub-wave's 16 lanes read consecutive slots); the direct loads fetched
 // the row once per sub-wave (64 / lpr times).  Without a slot (rows too long
 // for the block's LDS), direct loads.
@@ -246,16 +251,10 @@ __device__ __forceinline__ void fetch_row(const float *src, uint32_t ff, int lan
         if ((uint32_t)j < nper) r.v[j] = s4[lane + 64 * j];
 }
 
-template <bool SLOTS>
-__device__ __forceinline__ void staged_row(float4 *slot, const float *src, uint32_t ff, int lane,
-                                           uint32_t cl, float *xr, const RowRegs *pre = nullptr) {
-    if constexpr (!SLOTS) {
-        XChunk X;
-        X.load(src, nullptr, cl);
-#pragma unroll
-        for (int j = 0; j < 32; j++) xr[j] = X.xr[j];
-        return;
-    }
+// Writes the row into the wave's slot, from the registers fetch_row filled or
+// from memory.
+__device__ __forceinline__ void stage_row(float4 *slot, const float *src, uint32_t ff, int lane,
+                                          bool pre, const RowRegs &rr) {
     const uint32_t C = ff / 32, n4 = ff / 4;
     if (pre) {
         f32x4v *s = reinterpret_cast<f32x4v *>(slot);
@@ -263,7 +262,7 @@ __device__ __forceinline__ void staged_row(float4 *slot, const float *src, uint3
 #pragma unroll
         for (int j = 0; j < kRowLoadsMax; j++) {
             const uint32_t w4 = lane + 64 * j;
-            if ((uint32_t)j < nper) s[(w4 % 8) * C + w4 / 8] = pre->v[j];
+            if ((uint32_t)j < nper) s[(w4 % 8) * C + w4 / 8] = rr.v[j];
         }
     } else {
         const float4 *s4 = reinterpret_cast<const float4 *>(src);
@@ -271,109 +270,139 @@ __device__ __forceinline__ void staged_row(float4 *slot, const float *src, uint3
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     __builtin_amdgcn_wave_barrier();
+}
+
+// Chunk c of the row into xr: from the slot, or from memory.
+template <bool SLOTS>
+__device__ __forceinline__ void row_chunk(const float4 *slot, const float *src, uint32_t ff, uint32_t c, float *xr) {
+    if constexpr (!SLOTS) {
+        XChunk X;
+        X.load(src, nullptr, c);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const float4 v = slot[i * C + cl];
-        xr[4 * i + 0] = v.x;
-        xr[4 * i + 1] = v.y;
-        xr[4 * i + 2] = v.z;
-        xr[4 * i + 3] = v.w;
+        for (int j = 0; j < 32; j++) xr[j] = X.xr[j];
+    } else {
+        const uint32_t C = ff / 32;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float4 v = slot[i * C + c];
+            xr[4 * i + 0] = v.x;
+            xr[4 * i + 1] = v.y;
+            xr[4 * i + 2] = v.z;
+            xr[4 * i + 3] = v.w;
+        }
     }
 }
 
-template <int BITS, int ST, int BS, bool SLOTS>
+// The products of one expert's down rows (or the shared expert's) with its
+// activation row `src`, added to acc times wk: every chunk's weight loads
+// issue before the first product.
+template <int BITS, int ST, bool SLOTS, int CPL>
+__device__ __forceinline__ void down_rows_dot(const WDesc &w, uint64_t row_base, uint32_t h, uint32_t ff,
+                                              const float *src, bool pre, const RowRegs &rr, uint32_t row0, uint32_t sub,
+                                              uint32_t cl, uint32_t lpr, float4 *slot, float wk, float *acc,
+                                              [[maybe_unused]] uint32_t stamp, [[maybe_unused]] int phase) {
+    constexpr int FR = down_rows<CPL>();
+    const uint32_t rpi = 64u / lpr, C = ff / 32;
+    uint64_t rows[FR];
+    bool ok[FR];
+#pragma unroll
+    for (int f = 0; f < FR; f++) {
+        const uint32_t r = row0 + f * rpi + sub;
+        ok[f] = r < h;
+        rows[f] = row_base + r;
+    }
+    LaneRows<BITS, ST, FR> L[CPL];
+#pragma unroll
+    for (int c = 0; c < CPL; c++) L[c].load(w, rows, ok, cl + c * lpr, C);
+    loads_issued();
+    MOE_STAMP(stamp, phase);
+    if constexpr (SLOTS) stage_row(slot, src, ff, (int)(threadIdx.x & 63), pre, rr);
+    float part[FR];
+#pragma unroll
+    for (int f = 0; f < FR; f++) part[f] = 0.f;
+#pragma unroll
+    for (int c = 0; c < CPL; c++) {
+        XChunk X;  // SwiGLU activations (no norm)
+        row_chunk<SLOTS>(slot, src, ff, cl + c * lpr, X.xr);
+        float p[FR];
+        L[c].dot(X.xr, X.finish(nullptr, 0.f, 0, 0), p);
+#pragma unroll
+        for (int f = 0; f < FR; f++) part[f] += p[f];
+    }
+#pragma unroll
+    for (int f = 0; f < FR; f++) acc[f] += part[f] * wk;
+}
+
+template <int BITS, int ST, int BS, bool SLOTS, int CPL>
 __device__ __forceinline__ void down_wave(const DecodeKArgs &a, uint32_t wv, uint32_t nw,
-                                          uint32_t row0, uint32_t sub, uint32_t cl, uint32_t rpi,
-                                          float4 *slot, float *acc_r, float *acc_s) {
+                                          uint32_t row0, uint32_t sub, uint32_t cl, float4 *slot,
+                                          float *acc_r, float *acc_s) {
     const uint32_t n_exp = a.k + (a.has_shared ? 1u : 0u);
-    const uint32_t C = a.ff / 32;
+    [[maybe_unused]] const uint32_t stamp = kStampDown + blockIdx.x * nw + wv;
 #pragma unroll
     for (int q = 0; q < kDownMaxPerWave; q++) {
         const uint32_t kk = wv + q * nw;
         if (kk >= n_exp) break;
-        uint64_t rows[kDownFR];
-        bool ok[kDownFR];
-        float part[kDownFR];
-        XChunk X;  // this expert's SwiGLU activations (no norm)
+        const bool pre = SLOTS && row_in_regs(a.ff);
         if (kk < a.k) {
             // the activation row does not depend on the expert id: its loads
             // issue behind the id's, before the wait for it
             const uint32_t e = a.ids[kk];
             const float wk = a.weights[kk];
-            const bool pre = SLOTS && row_in_regs(a.ff);
+            const float *src = a.act + (uint64_t)kk * a.ff;
             RowRegs rr;
-            if (pre) fetch_row(a.act + (uint64_t)kk * a.ff, a.ff, (int)(threadIdx.x & 63), rr);
-#pragma unroll
-            for (int f = 0; f < kDownFR; f++) {
-                const uint32_t r = row0 + f * rpi + sub;
-                ok[f] = r < a.h;
-                rows[f] = (uint64_t)e * a.h + r;
-            }
-            LaneRows<BITS, ST, kDownFR> L;
-            L.load(a.down, rows, ok, cl, C);
-            loads_issued();
-            MOE_STAMP(kStampDown + blockIdx.x * nw + wv, 1 + q);
-            staged_row<SLOTS>(slot, a.act + (uint64_t)kk * a.ff, a.ff, (int)(threadIdx.x & 63), cl, X.xr,
-                              pre ? &rr : nullptr);
-            L.dot(X.xr, X.finish(nullptr, 0.f, 0, 0), part);
-#pragma unroll
-            for (int f = 0; f < kDownFR; f++) acc_r[f] += part[f] * wk;
+            if (pre) fetch_row(src, a.ff, (int)(threadIdx.x & 63), rr);
+            down_rows_dot<BITS, ST, SLOTS, CPL>(a.down, (uint64_t)e * a.h, a.h, a.ff, src, pre, rr, row0, sub, cl,
+                                                a.lpr_f, slot, wk, acc_r, stamp, 1 + q);
         } else {
-            const bool pre = SLOTS && row_in_regs(a.ff);
             RowRegs rr;
             if (pre) fetch_row(a.sh_act, a.ff, (int)(threadIdx.x & 63), rr);
-#pragma unroll
-            for (int f = 0; f < kDownFR; f++) {
-                const uint32_t r = row0 + f * rpi + sub;
-                ok[f] = r < a.h;
-                rows[f] = r;
-            }
-            LaneRows<BS, ST, kDownFR> L;
-            L.load(a.sd, rows, ok, cl, C);
-            loads_issued();
-            staged_row<SLOTS>(slot, a.sh_act, a.ff, (int)(threadIdx.x & 63), cl, X.xr, pre ? &rr : nullptr);
-            L.dot(X.xr, X.finish(nullptr, 0.f, 0, 0), part);
-#pragma unroll
-            for (int f = 0; f < kDownFR; f++) acc_s[f] += part[f];
+            down_rows_dot<BS, ST, SLOTS, CPL>(a.sd, 0, a.h, a.ff, a.sh_act, pre, rr, row0, sub, cl, a.lpr_f, slot,
+                                              1.0f, acc_s, stamp, 1 + q);
         }
     }
 }
 
-template <int BITS, int ST, bool SLOTS>
+template <int BITS, int ST, bool SLOTS, int CPL>
 __global__ __launch_bounds__(64 * kDownMaxWaves) void decode_down_kernel(DecodeKArgs a) {
+    constexpr int FR = down_rows<CPL>();
     __shared__ float red_r[kDownMaxWaves][128];
     __shared__ float red_s[kDownMaxWaves][128];
     extern __shared__ float4 dslot[];  // [waves][ff / 4] with SLOTS
     const int lane = threadIdx.x & 63;
     const uint32_t wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
     const uint32_t lpr = a.lpr_f, rpi = 64u / lpr, sub = lane / lpr, cl = lane % lpr;
-    const uint32_t rows_per_block = rpi * kDownFR;
+    const uint32_t rows_per_block = rpi * FR;
     const uint32_t row0 = blockIdx.x * rows_per_block;
     float4 *slot = SLOTS ? dslot + wv * (a.ff / 4) : nullptr;
     const uint32_t stamp = kStampDown + blockIdx.x * nw + wv;
     MOE_STAMP(stamp, 0);
     // issued first: needed only after the LDS combine
     const float shared_gate = a.has_shared ? a.sh_gate[0] : 0.f;
-    float acc_r[kDownFR], acc_s[kDownFR];
+    float acc_r[FR], acc_s[FR];
 #pragma unroll
-    for (int f = 0; f < kDownFR; f++) acc_r[f] = acc_s[f] = 0.f;
+    for (int f = 0; f < FR; f++) acc_r[f] = acc_s[f] = 0.f;
     switch (a.has_shared ? a.sd.bits : BITS) {
-    case 2: down_wave<BITS, ST, 2, SLOTS>(a, wv, nw, row0, sub, cl, rpi, slot, acc_r, acc_s); break;
-    case 4: down_wave<BITS, ST, 4, SLOTS>(a, wv, nw, row0, sub, cl, rpi, slot, acc_r, acc_s); break;
-    default: down_wave<BITS, ST, 8, SLOTS>(a, wv, nw, row0, sub, cl, rpi, slot, acc_r, acc_s); break;
+    case 2: down_wave<BITS, ST, 2, SLOTS, CPL>(a, wv, nw, row0, sub, cl, slot, acc_r, acc_s); break;
+    case 4: down_wave<BITS, ST, 4, SLOTS, CPL>(a, wv, nw, row0, sub, cl, slot, acc_r, acc_s); break;
+    default: down_wave<BITS, ST, 8, SLOTS, CPL>(a, wv, nw, row0, sub, cl, slot, acc_r, acc_s); break;
     }
     MOE_STAMP(stamp, 3);
-    static_assert(kDownFR == 2, "reduce-scatter layout assumes two rows per sub-wave");
-    if (lpr >= 16) {
-        float r, sh;
-        rs2_pairs(acc_r, acc_s, lane, lpr, r, sh);
-        if (cl < 2) {
-            red_r[wv][cl * rpi + sub] = r;
-            red_s[wv][cl * rpi + sub] = sh;
+    bool scattered = false;
+    if constexpr (FR == 2) {  // the reduce-scatter takes two rows per sub-wave
+        if (lpr >= 16) {
+            float r, sh;
+            rs2_pairs(acc_r, acc_s, lane, lpr, r, sh);
+            if (cl < 2) {
+                red_r[wv][cl * rpi + sub] = r;
+                red_s[wv][cl * rpi + sub] = sh;
+            }
+            scattered = true;
         }
-    } else {
+    }
+    if (!scattered) {
 #pragma unroll
-        for (int f = 0; f < kDownFR; f++) {
+        for (int f = 0; f < FR; f++) {
             const float r = subwave_sum(acc_r[f], (int)lpr), sh = subwave_sum(acc_s[f], (int)lpr);
             if (cl == 0) {
                 red_r[wv][f * rpi + sub] = r;
@@ -407,6 +436,15 @@ static bool pow2_chunks(uint32_t n) {
     const uint32_t c = n / 32;
     return c >= 1 && c <= 64 && (c & (c - 1)) == 0;
 }
+// Rows of ff values: 2^k or 3 * 2^k chunks of 32, at most 64 lanes of one or
+// three chunks (0: neither; those layers take the grouped path).  With three
+// chunks a lane the 128-expert layer of ff 768 decodes in 18.3 us (decode_down
+// 4.7), against 104 on the grouped path, whose wave walks one row at a time
+// with a load per word in flight.
+static uint32_t down_chunks_per_lane(uint32_t ff) {
+    if (pow2_chunks(ff)) return 1;
+    return ff % 3 == 0 && pow2_chunks(ff / 3) ? 3 : 0;
+}
 static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 bool decode_supported(const DecodeArgs &a) {
@@ -414,7 +452,7 @@ bool decode_supported(const DecodeArgs &a) {
     if (g.bits == 0 || a.up.bits != g.bits || a.down.bits != g.bits) return false;
     if (a.up.type != g.type || a.down.type != g.type) return false;
     const uint32_t st = g.type;
-    if (!pow2_chunks(g.in) || !pow2_chunks(g.out)) return false;
+    if (!pow2_chunks(g.in) || !down_chunks_per_lane(g.out)) return false;
     if (a.router.bits && a.router.type != st) return false;
     if (a.router.out > 4096 || a.k == 0 || a.k > 64 || a.k > a.router.out) return false;
     // the down kernel covers at most kDownMaxWaves * kDownMaxPerWave experts
@@ -434,6 +472,19 @@ bool decode_supported(const DecodeArgs &a) {
     return true;
 }
 
+template <int BITS, int ST, int CPL>
+static hipError_t launch_down(Prof *p, hipStream_t s, const DecodeKArgs &k) {
+    const uint32_t rows_per_block = (64u / k.lpr_f) * down_rows<CPL>();
+    const uint32_t n_exp = k.k + (k.has_shared ? 1u : 0u);
+    const uint32_t nw = n_exp < (uint32_t)kDownMaxWaves ? n_exp : (uint32_t)kDownMaxWaves;
+    // one activation-row slot per wave when they fit beside the combine arrays
+    const size_t slots = (size_t)nw * k.ff * 4;
+    const dim3 grid((k.h + rows_per_block - 1) / rows_per_block), block(64 * nw);
+    if (slots <= kDownSlotBytes)
+        return launch_kernel(p, "decode_down", decode_down_kernel<BITS, ST, true, CPL>, grid, block, slots, s, k);
+    return launch_kernel(p, "decode_down", decode_down_kernel<BITS, ST, false, CPL>, grid, block, 0, s, k);
+}
+
 template <int BITS, int ST>
 static hipError_t launch_decode_t(Prof *p, hipStream_t s, const DecodeKArgs &k) {
     const uint32_t pre_waves = k.n_router_waves + (k.has_shared ? 1 : 0);
@@ -446,15 +497,7 @@ static hipError_t launch_decode_t(Prof *p, hipStream_t s, const DecodeKArgs &k) 
     e = launch_kernel(p, "decode_gateup", decode_gateup_kernel<BITS, ST>, dim3(gate_waves), dim3(64),
                       lds, s, k);
     if (e != hipSuccess) return e;
-    const uint32_t rows_per_block = (64u / k.lpr_f) * kDownFR;
-    const uint32_t n_exp = k.k + (k.has_shared ? 1u : 0u);
-    const uint32_t nw = n_exp < (uint32_t)kDownMaxWaves ? n_exp : (uint32_t)kDownMaxWaves;
-    // one activation-row slot per wave when they fit beside the combine arrays
-    const size_t slots = (size_t)nw * k.ff * 4;
-    const dim3 grid((k.h + rows_per_block - 1) / rows_per_block), block(64 * nw);
-    if (slots <= kDownSlotBytes)
-        return launch_kernel(p, "decode_down", decode_down_kernel<BITS, ST, true>, grid, block, slots, s, k);
-    return launch_kernel(p, "decode_down", decode_down_kernel<BITS, ST, false>, grid, block, 0, s, k);
+    return k.ff / 32 == k.lpr_f ? launch_down<BITS, ST, 1>(p, s, k) : launch_down<BITS, ST, 3>(p, s, k);
 }
 
 hipError_t launch_decode(Prof *p, hipStream_t s, const DecodeArgs &a) {
@@ -463,7 +506,7 @@ hipError_t launch_decode(Prof *p, hipStream_t s, const DecodeArgs &a) {
     k.sg = a.sg; k.su = a.su; k.sd = a.sd; k.sgi = a.sgi;
     k.has_shared = a.has_shared; k.k = a.k; k.normalize = a.normalize;
     k.h = a.gate.in; k.ff = a.gate.out; k.ffs = a.has_shared ? a.sg.out : 0; k.E = a.router.out;
-    k.lpr_h = k.h / 32; k.lpr_f = k.ff / 32;
+    k.lpr_h = k.h / 32; k.lpr_f = k.ff / 32 / down_chunks_per_lane(k.ff);
     const uint32_t rpi_h = 64u / k.lpr_h;
     k.n_router_waves = (k.E + rpi_h * kPreFR - 1) / (rpi_h * kPreFR);
     k.n_shared_waves = (k.ffs + rpi_h * kGateFR - 1) / (rpi_h * kGateFR);

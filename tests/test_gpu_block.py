@@ -387,6 +387,25 @@ def test_decode_long_down_rows(gpu, shared):
         assert rel_max_err(got[0], ref[0]) <= F32_TOL
 
 
+@pytest.mark.parametrize("ff,shared,kind", [(96, 0, (4, 32, BF16)), (192, 192, (8, 64, F16)), (768, 0, (4, 64, BF16)),
+                                            (768, 768, (2, 32, BF16)), (1536, 1536, (8, 128, F32)),
+                                            (3072, 0, (4, 128, BF16))])
+def test_decode_three_chunk_down_rows(gpu, ff, shared, kind):
+    """Fused decode with down rows of 3 * 2^k chunks of 32 (Qwen3-30B-A3B's ff
+    768): every lane owns three chunks of its row.  One lane per row (96) to 32
+    (3072), activation slots written from registers, by the general loop and
+    not at all (3072), with and without a shared expert."""
+    print(f"[case] decode ff={ff} shared={shared} kind={kind}", flush=True)
+    kinds = {"router": DENSE, "experts": kind, "shared": kind, "shared_gate": DENSE}
+    blk = HostBlock(256, 16, 8, ff, shared, kinds, seed=ff + shared, random_experts=True)
+    bw = blk.upload(gpu)
+    for seed in range(2):
+        x = synth.normal(5120 + seed, 256).reshape(1, 256)
+        got, prof = profiled(gpu, lambda: run_block(gpu, bw, x, 1, PATH_AUTO))
+        assert "decode_down" in prof, sorted(prof)
+        check_against_oracle(blk, x, got)
+
+
 @pytest.mark.parametrize("E,shared", [(1100, 0), (1100, 128)])
 def test_decode_many_experts(gpu, E, shared):
     """The fused decode past 1024 experts, where every routing wave keeps the
