@@ -823,6 +823,22 @@ def test_mfma_bf16_input_copy(gpu, c4, norm):
         assert diff.max() <= 1, diff.max()
 
 
+@pytest.mark.parametrize("E,h,T", [(30, 256, 130), (36, 1024, 130), (33, 2048, 140)])
+def test_router_partial_sums(gpu, E, h, T):
+    """The F32 router's partial sums of 2 to 16 K ranges (one to two groups of
+    the loads in flight) summed and routed, over logit rows that are and are not
+    a multiple of four: logits, ids and weights against the oracle."""
+    print(f"[case] router partial sums E={E} h={h} T={T}", flush=True)
+    kinds = {"router": DENSE, "experts": (4, 64, BF16)}
+    blk = HostBlock(h, E, 4, 128, 0, kinds, seed=E, random_experts=True)
+    bw = blk.upload(gpu)
+    x = synth.normal(4800 + E, T * h).reshape(T, h)
+    bias = zipf_bias(T, E, E)
+    got = run_block(gpu, bw, x, T, PATH_MFMA, bias=bias)
+    check_all_ids(blk, got)
+    check_against_oracle(blk, x, got, bias=bias, tol=BF16_TOL)
+
+
 def test_config4_routing_matches_oracle_f32_logits(gpu, c4):
     """The prefill path routes on F32 router products: its logits of all
     4096 tokens agree with the oracle's own F32 logits (orc_matmul, the
