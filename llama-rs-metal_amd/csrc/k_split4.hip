@@ -1,0 +1,11 @@
+// The split products (split_mm.hpp) over 4-bit codes, in a translation unit
+// of their own so the code widths compile beside each other.
+#include "split_mm.hpp"
+
+namespace moehip {
+
+hipError_t split::launch4(const Launch &l, int mode) {
+    return mode == GATEUP ? l.kind<GATEUP, 4>() : l.kind<ROWS, 4>();
+}
+
+}  // namespace moehip

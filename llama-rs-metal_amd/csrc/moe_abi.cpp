@@ -291,7 +291,14 @@ moe_status moe_matmul(moe_gpu *g, const moe_weight *w, moe_buffer x, moe_buffer 
     if ((st = check_alias(g, reads, {rng(y)}, false))) return st;
     WDesc d = wdesc(*w);
     // 4 tokens or more: a tiled F32 product, as the reference switches to
-    // affine_mm / gemm_simd (matrix.rs:77-123); fewer: one GEMV per token
+    // affine_mm / gemm_simd (matrix.rs:77-123); fewer: one GEMV per token.
+    // Affine weights as split products on the f16 matrix cores (h 2048 -> 4096
+    // 4-bit rows at 4 / 256 / 2000 tokens 12 / 26 / 144 us, on the F32 matrix
+    // cores 47 / 52 / 280, and a fifth of their error), the rest on the F32 ones
+    if (tokens >= 4 && split_supported(d, (const float *)x.ptr))
+        return launched(g, launch_split_rows(&g->prof, g->stream, "matmul_f32", d, (const float *)x.ptr, nullptr,
+                                             nullptr, nullptr, (uint32_t)tokens, 0, nullptr, (float *)y.ptr),
+                        "matmul");
     if (tokens >= 4 && f32mm_supported(d, (const float *)x.ptr))
         return launched(g, launch_f32mm(&g->prof, g->stream, "matmul_f32", d, (const float *)x.ptr,
                                         (uint32_t)tokens, 1, nullptr, (float *)y.ptr),

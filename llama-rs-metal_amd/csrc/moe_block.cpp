@@ -250,21 +250,21 @@ moe_status run_grouped(moe_gpu *g, const moe_block_weights *w, const Dims &d, co
     return MOE_OK;
 }
 
-// Batched decode (k_batched.hip): several tokens whose expert segments are
-// too short for the MFMA path.  Same composition as run_grouped; every
-// product streams its weight rows once per run of seg_tokens() inputs.
+// Batched decode: several tokens whose expert segments are too short for the
+// bf16 MFMA path.  Same composition as run_grouped; every product streams its
+// weight rows once per entry of a few input rows, on VALU (k_batched.hip) or,
+// for affine weights, as split products on the f16 matrix cores (k_split.hip).
+bool split_ok(const WDesc &w) { return split_supported(w, nullptr); }
+bool rows_ok(const WDesc &w) { return seg_supported(w) || split_ok(w); }
+bool gateup_ok(const WDesc &g, const WDesc &u) {
+    return g.bits == u.bits && g.type == u.type &&
+           ((seg_supported(g) && seg_supported(u)) || (split_ok(g) && split_ok(u) && g.gshift == u.gshift));
+}
 bool batched_ok(const moe_block_weights *w) {
-    const WDesc G = wdesc(w->gate), U = wdesc(w->up), D = wdesc(w->down);
-    if (!seg_supported(wdesc(w->router)) || !seg_supported(G) || !seg_supported(U) ||
-        !seg_supported(D) || G.bits != U.bits || G.type != U.type)
+    if (!rows_ok(wdesc(w->router)) || !gateup_ok(wdesc(w->gate), wdesc(w->up)) || !rows_ok(wdesc(w->down)))
         return false;
-    if (w->has_shared) {
-        const WDesc SG = wdesc(w->shared_gate), SU = wdesc(w->shared_up);
-        if (!seg_supported(SG) || !seg_supported(SU) || !seg_supported(wdesc(w->shared_down)) ||
-            !seg_supported(gate_inp_desc(w->shared_gate_inp)) || SG.bits != SU.bits ||
-            SG.type != SU.type)
-            return false;
-    }
+    if (w->has_shared)
+        return gateup_ok(wdesc(w->shared_gate), wdesc(w->shared_up)) && rows_ok(wdesc(w->shared_down));
     return true;
 }
 
@@ -281,8 +281,28 @@ moe_status run_batched(moe_gpu *g, const moe_block_weights *w, const Dims &d, co
     uint32_t *tiles = reinterpret_cast<uint32_t *>(ws + L.tiles);
     uint32_t *ntiles = reinterpret_cast<uint32_t *>(ws + L.ntiles);
     float *act = ws + L.act, *yexp = ws + L.yexp;
-    const uint32_t runs = seg_max_entries(t32, 0), entries = seg_max_entries(t32 * K, E);
+    const uint32_t entries = seg_max_entries(t32 * K, E);
     const float *bias = has(io->logit_bias) ? fp(io->logit_bias) : nullptr;
+    // Products over all tokens (router, shared expert) and over the dispatched
+    // segments, each on VALU or as split products
+    auto rows = [&](hipStream_t st, const char *name, const WDesc &W, const float *in, bool segs, const float *b,
+                    float *o) {
+        const uint32_t n = segs ? t32 * K : t32;
+        const bool split = split_ok(W) && (!seg_supported(W) || split_rows_better(W, n, segs ? E : 1));
+        const uint32_t *tl = segs ? tiles : nullptr, *nt = segs ? ntiles : nullptr, *of = segs ? offsets : nullptr;
+        if (split) return launch_split_rows(p, st, name, W, in, tl, nt, of, n, entries, b, o);
+        return launch_seg_rows(p, st, name, W, in, tl, nt, of, segs ? 0 : n, segs ? entries : seg_max_entries(n, 0), b, o);
+    };
+    auto gateup = [&](hipStream_t st, const char *name, const WDesc &G, const WDesc &U, bool segs, float *o) {
+        const uint32_t n = segs ? t32 * K : t32;
+        const bool split = split_ok(G) && split_ok(U) && G.gshift == U.gshift &&
+                           (!seg_supported(G) || split_rows_better(G, n, segs ? E : 1));
+        const uint32_t *tl = segs ? tiles : nullptr, *nt = segs ? ntiles : nullptr, *of = segs ? offsets : nullptr;
+        const uint32_t *pm = segs ? perm : nullptr;
+        if (split) return launch_split_gateup(p, st, name, G, U, xin, pm, segs ? K : 1, tl, nt, of, n, entries, o);
+        return launch_seg_gateup(p, st, name, G, U, xin, pm, segs ? K : 1, tl, nt, of, segs ? 0 : n,
+                                 segs ? entries : seg_max_entries(n, 0), o);
+    };
     // the shared expert needs only the input: it runs on the side stream,
     // concurrently with the routed chain, and joins before the combine.  Its
     // fork point precedes the router, but the router is queued first: a
@@ -292,32 +312,39 @@ moe_status run_batched(moe_gpu *g, const moe_block_weights *w, const Dims &d, co
     const float *so = nullptr, *sgv = nullptr;
     SideFork side{g, s};
     if (w->has_shared) TRY(side.mark());
-    TRY(launch_seg_rows(p, s, "seg_router", wdesc(w->router), xin, nullptr, nullptr, nullptr, t32, runs,
-                        bias, logits));
+    // A router of many logits: the F32 matrix cores (K split over the grid, its
+    // partial sums in y16, which this path leaves idle), from 2^15 logits on:
+    // 512 dense rows at 64 / 500 tokens 9 / 21 us against 17 / 258 on VALU
+    const WDesc R = wdesc(w->router);
+    const bool f32_router = (uint64_t)t32 * E >= (1u << 15) && f32mm_supported(R, xin);
+    const uint32_t rks = f32_router ? f32mm_ksplit(R, t32, (uint64_t)T * K * d.h / 2) : 1;
+    float *parts = ws + L.y16;
+    if (f32_router)
+        TRY(launch_f32mm(p, s, "seg_router", R, xin, t32, rks, rks > 1 ? nullptr : bias, rks > 1 ? parts : logits));
+    else
+        TRY(rows(s, "seg_router", R, xin, false, bias, logits));
     if (w->has_shared) {
         float *sh = ws + L.sh_act, *sout = ws + L.sh_out, *sgt = ws + L.sh_gate;
         hipStream_t ss = g->side;
         TRY(side.enter());
-        TRY(launch_seg_gateup(p, ss, "seg_shared_gateup", wdesc(w->shared_gate), wdesc(w->shared_up), xin,
-                              nullptr, 1, nullptr, nullptr, nullptr, t32, runs, sh));
-        TRY(launch_seg_rows(p, ss, "seg_shared_down", wdesc(w->shared_down), sh, nullptr, nullptr, nullptr,
-                            t32, runs, nullptr, sout));
-        TRY(launch_seg_rows(p, ss, "seg_shared_gate", gate_inp_desc(w->shared_gate_inp), xin, nullptr,
-                            nullptr, nullptr, t32, runs, nullptr, sgt));
+        TRY(gateup(ss, "seg_shared_gateup", wdesc(w->shared_gate), wdesc(w->shared_up), false, sh));
+        TRY(rows(ss, "seg_shared_down", wdesc(w->shared_down), sh, false, nullptr, sout));
+        TRY(launch_gemv(p, ss, gate_inp_desc(w->shared_gate_inp), xin, 0, nullptr, 1, sgt, t32));
         so = sout;
         sgv = sgt;
     }
-    if (route_dispatch_fits(E, K, t32)) {
+    if (rks > 1) {
+        TRY(launch_route_sum(p, s, parts, rks, bias, E, K, w->normalize ? 1 : 0, t32, logits, ids, wts));
+        TRY(launch_dispatch(p, s, ids, t32 * K, E, counts, offsets, perm, pos, seg_tokens(), tiles, ntiles));
+    } else if (route_dispatch_fits(E, K, t32)) {
         TRY(launch_route_dispatch(p, s, logits, E, K, w->normalize ? 1 : 0, t32, ids, wts, g->arrive,
                                   seg_tokens(), counts, offsets, perm, pos, tiles, ntiles));
     } else {
         TRY(launch_route(p, s, logits, E, K, w->normalize ? 1 : 0, t32, ids, wts));
         TRY(launch_dispatch(p, s, ids, t32 * K, E, counts, offsets, perm, pos, seg_tokens(), tiles, ntiles));
     }
-    TRY(launch_seg_gateup(p, s, "seg_gateup", wdesc(w->gate), wdesc(w->up), xin, perm, K, tiles, ntiles,
-                          offsets, 0, entries, act));
-    TRY(launch_seg_rows(p, s, "seg_down", wdesc(w->down), act, tiles, ntiles, offsets, 0, entries,
-                        nullptr, yexp));
+    TRY(gateup(s, "seg_gateup", wdesc(w->gate), wdesc(w->up), true, act));
+    TRY(rows(s, "seg_down", wdesc(w->down), act, true, nullptr, yexp));
     TRY(side.join());
     TRY(launch_combine(p, s, yexp, pos, wts, K, so, sgv, io->residual ? xres : nullptr, out, t32,
                        (uint32_t)d.h));

@@ -236,6 +236,18 @@ hipError_t launch_seg_rows(Prof *p, hipStream_t s, const char *name, const WDesc
                            const float *in, const uint32_t *tiles, const uint32_t *ntiles,
                            const uint32_t *offsets, uint32_t n, uint32_t entries, const float *bias,
                            float *out);
+// ---- F32-accurate products of affine weights on the f16 matrix cores (k_split*.hip) ----
+// The same products and work entries as launch_seg_gateup / launch_seg_rows.
+bool split_supported(const WDesc &w, const float *x);  // affine, whole units of 128 values, 16-byte aligned
+// whether the split products beat the VALU rows for n input rows over `experts`
+bool split_rows_better(const WDesc &w, uint32_t n, uint32_t experts);
+hipError_t launch_split_gateup(Prof *p, hipStream_t s, const char *name, const WDesc &gate, const WDesc &up,
+                               const float *x, const uint32_t *perm, uint32_t k, const uint32_t *tiles,
+                               const uint32_t *ntiles, const uint32_t *offsets, uint32_t n, uint32_t entries,
+                               float *act);
+hipError_t launch_split_rows(Prof *p, hipStream_t s, const char *name, const WDesc &w, const float *in,
+                             const uint32_t *tiles, const uint32_t *ntiles, const uint32_t *offsets, uint32_t n,
+                             uint32_t entries, const float *bias, float *out);
 // (expert, first position) of every run of `tm` pairs of the non-empty
 // segments, and their count (k_mfma.hip)
 hipError_t launch_tile_schedule(Prof *p, hipStream_t s, const uint32_t *offsets, uint32_t experts,

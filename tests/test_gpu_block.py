@@ -347,6 +347,29 @@ def test_batched_decode_layouts(gpu, experts, T):
     assert rel_max_err(got[0], ref[0]) <= F32_TOL
 
 
+@pytest.mark.parametrize("experts", [(2, 32, BF16), (4, 64, F16), (4, 128, F32), (8, 32, BF16), (8, 128, F16)])
+@pytest.mark.parametrize("ff,ffs,T", [(128, 128, 30), (384, 0, 17), (384, 256, 100)])
+def test_batched_split_products(gpu, experts, ff, ffs, T):
+    """The batched decode where the expert segments are long enough for the
+    split products (and, with ff 384, where the VALU rows do not take the down
+    rows at any length): ragged segments of 0 to over 32 pairs, segments that
+    end inside and at a 16-pair entry, the shared expert on either side of its
+    own threshold, every code width; and the router's F32 matrix-core product
+    where it has enough logits."""
+    print(f"[case] batched split experts={experts} ff={ff} ffs={ffs} T={T}", flush=True)
+    E = 48 if T < 100 else 400
+    kinds = {"router": (8, 64, BF16), "experts": experts, "shared": (4, 64, BF16), "shared_gate": DENSE}
+    blk = HostBlock(256, E, 4, ff, ffs, kinds, seed=60 + T + ff, random_experts=True)
+    bw = blk.upload(gpu)
+    x = synth.normal(4650 + T, T * 256).reshape(T, 256)
+    bias = hot_bias(T, E, seed=T, frac=0.5, hot=5, boost=4.0)
+    wsd = {}
+    got = run_block(gpu, bw, x, T, PATH_AUTO, bias=bias, ws_out=wsd)
+    check_all_ids(blk, got)
+    check_against_oracle(blk, x, got, bias=bias)
+    check_in_block_dispatch(bw, T, got[2], wsd["ws"], tm=bw.workspace_layout(T)["tile_pairs_batched"])
+
+
 def test_route_dispatch_grids_in_sequence(gpu):
     """The fused route + dispatch launch counts its finished blocks on a
     device word that its last block puts back to zero: launches of 1, 18, 2

@@ -359,3 +359,67 @@ def test_norm_rows(gpu, n, heads, pad, dtype):
             close(got[i], oracle.rms_norm(row, wf, 1e-5), 2e-4)
         gpu.release(y)
     gpu.release(buf)
+
+
+@pytest.mark.parametrize("bits,group,st", [(2, 32, F32), (2, 64, BF16), (2, 128, F16), (4, 32, BF16), (4, 64, F16),
+                                           (4, 128, F32), (8, 32, F16), (8, 64, F32), (8, 128, BF16)])
+@pytest.mark.parametrize("n_in,out,tokens", [(128, 1, 4), (256, 17, 15), (384, 130, 16), (512, 64, 17), (640, 255, 33),
+                                             (1152, 1040, 500)])
+def test_matmul_split_products(gpu, bits, group, st, n_in, out, tokens):
+    """Batch::matmul of affine weights from 4 tokens on (split f16 products) at
+    the edges of its tiles: one to nine units of 128 values, output rows and
+    tokens around 16, both tile counts per wave, over rows of unlike magnitude
+    (2^-30 .. 2^30, one of zeros).  The bound per output is that of the method:
+    2^-22 of each product (the split of x) and F32 additions of one sum per
+    group, under 2^-20 * sum |w x| together."""
+    print(f"[case] split {bits}/{group}/{st} [{n_in},{out}] tokens={tokens}", flush=True)
+    q = synth.quantize_affine(synth.normal(31 * n_in + bits, n_in * out, 0.0, 0.5), bits, group, st)
+    t = Tensor.affine([n_in, out], *q, bits, group, st)
+    x = synth.normal(32 * n_in + tokens, tokens * n_in).reshape(tokens, n_in)
+    x = (x * np.exp2(np.linspace(-30, 30, tokens))[:, None]).astype(np.float32)
+    x[tokens // 2] = 0.0
+    w = gpu.weight_tensor(t)
+    xb, y = gpu.upload(x), gpu.zeros(tokens * out)
+    with gpu.batch() as b:
+        b.matmul(w, xb, y, tokens)
+    got = gpu.read(y).reshape(tokens, out).astype(np.float64)
+    wd = np.asarray(oracle.decode(t), np.float64).reshape(out, n_in)
+    ref, mag = x.astype(np.float64) @ wd.T, np.abs(x.astype(np.float64)) @ np.abs(wd).T
+    assert np.all(np.abs(got - ref) <= 2.0 ** -20 * mag)
+    for b_ in (xb, y):
+        gpu.release(b_)
+
+
+def test_matmul_split_nonfinite_rows(gpu):
+    """A NaN or an infinity in a token's row reaches every output of that token
+    and of no other."""
+    t = Tensor.affine([256, 40], *synth.quantize_affine(synth.normal(5, 256 * 40), 4, 64, BF16), 4, 64, BF16)
+    x = synth.normal(6, 6 * 256).reshape(6, 256)
+    x[1, 200], x[3, 7], x[4, 8] = np.nan, np.inf, -np.inf
+    w, xb, y = gpu.weight_tensor(t), gpu.upload(x), gpu.zeros(6 * 40)
+    with gpu.batch() as b:
+        b.matmul(w, xb, y, 6)
+    got = gpu.read(y).reshape(6, 40)
+    for i in (1, 3, 4):
+        assert not np.isfinite(got[i]).any()
+    for i in (0, 2, 5):
+        assert np.isfinite(got[i]).all()
+    for b_ in (xb, y):
+        gpu.release(b_)
+
+
+def test_matmul_split_long_runs(gpu):
+    """More token rows than one launch's grid holds (65535 entries of 16): the
+    rows on both sides of the boundary and the last ones."""
+    n_in, out, tokens = 128, 3, 65535 * 16 + 21
+    t = Tensor.affine([n_in, out], *synth.quantize_affine(synth.normal(8, n_in * out), 4, 64, BF16), 4, 64, BF16)
+    base = synth.normal(9, 997 * n_in).reshape(997, n_in)
+    x = np.resize(base, (tokens, n_in))
+    w, xb, y = gpu.weight_tensor(t), gpu.upload(x), gpu.zeros(tokens * out)
+    with gpu.batch() as b:
+        b.matmul(w, xb, y, tokens)
+    got = gpu.read(y).reshape(tokens, out)
+    ref = oracle.matmul(t, base, 997).reshape(997, out)
+    close(got, np.resize(ref, (tokens, out)))
+    for b_ in (xb, y):
+        gpu.release(b_)
