@@ -16,19 +16,20 @@ namespace moehip {
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-// Sums of 32 values over their four runs of eight.
+// Sums of 32 values over their runs of L.
+template <int L>
 __device__ __forceinline__ void run_sums(const float *x, float *rs) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        rs[i] = x[8 * i];
+    for (int i = 0; i < 32 / L; i++) {
+        rs[i] = x[L * i];
 #pragma unroll
-        for (int j = 1; j < 8; j++) rs[i] += x[8 * i + j];
+        for (int j = 1; j < L; j++) rs[i] += x[L * i + j];
     }
 }
 __device__ __forceinline__ float sum32(const float *x) {
-    float rs[4];
-    run_sums(x, rs);
-    return (rs[0] + rs[1]) + (rs[2] + rs[3]);
+    float rs[8];
+    run_sums<4>(x, rs);
+    return ((rs[0] + rs[1]) + (rs[2] + rs[3])) + ((rs[4] + rs[5]) + (rs[6] + rs[7]));
 }
 
 // 32 consecutive weight elements of one row as raw words.
@@ -56,14 +57,16 @@ struct Chunk32 {
     }
     // sum_j value_j * x[j]; for affine rows value_j is the centred code
     // (code - kCentre), so that the sum and its rounding stay small.  rs: the
-    // sums of x over its four runs of eight (run_sums; affine rows only).
+    // sums of x over its runs of kRun (run_sums; affine rows only).
     // F16 = false: each run's chain of FMAs over the unsigned codes starts at
-    // -kCentre times the run's sum.  The shortest code (4-byte conversions and
-    // FMAs), for waves that run through their rows once: decode_gateup 7.7 us
-    // against 8.5 with F16.
+    // -kCentre times the run's sum (shorter runs at 8 bits, whose centre is the
+    // larger against what the sum comes to).  The shortest code (4-byte
+    // conversions and FMAs), for waves that run through their rows once:
+    // decode_gateup 7.7 us against 8.5 with F16.
     // F16 = true: eight codes at a time to centred f16 (codes16.hpp),
     // multiplied by mixed-precision FMAs: fewer instructions, for waves whose
     // arithmetic repeats over inputs (seg_down at 64 tokens 90 -> 68 us).
+    static constexpr int kRun = BITS == 8 ? 4 : 8;
     static constexpr float kCentre = BITS ? (float)(1 << (BITS ? BITS - 1 : 0)) : 0.f;
     template <bool F16>
     __device__ __forceinline__ float dot(const float *x, [[maybe_unused]] const float *rs) const {
@@ -83,19 +86,18 @@ struct Chunk32 {
                 d += r;
             }
         } else if constexpr (BITS) {
-            constexpr int P = 32 / BITS;               // codes per word
-            constexpr int RW = P > 8 ? P / 8 : 1;      // runs per word, or
-            constexpr int WR = P < 8 ? 8 / P : 1;      // words per run
+            constexpr int P = 32 / BITS;     // codes per word
+            constexpr int RW = P / kRun;     // runs per word
 #pragma unroll
-            for (int i = 0; i < 4; i += RW) {
-                float c[8 * RW];
-#pragma unroll
-                for (int k = 0; k < WR; k++) unpack_word<BITS>(w[i * WR / RW + k], c + k * P);
+            for (int i = 0; i < NW; i++) {
+                float c[P];
+                unpack_word<BITS>(w[i], c);
 #pragma unroll
                 for (int k = 0; k < RW; k++) {
-                    float r = -kCentre * rs[i + k];
+                    const int n = RW * i + k;
+                    float r = -kCentre * rs[n];
 #pragma unroll
-                    for (int j = 0; j < 8; j++) r = fmaf(c[8 * k + j], x[8 * (i + k) + j], r);
+                    for (int j = 0; j < kRun; j++) r = fmaf(c[kRun * k + j], x[kRun * n + j], r);
                     d += r;
                 }
             }
@@ -151,8 +153,8 @@ struct LaneRows {
     }
     template <bool F16 = false>
     __device__ __forceinline__ void dot(const float *x, float xsum, float *res) const {
-        float rs[4];
-        if constexpr (BITS && !F16) run_sums(x, rs);
+        float rs[32 / Chunk32<BITS, T>::kRun];
+        if constexpr (BITS && !F16) run_sums<Chunk32<BITS, T>::kRun>(x, rs);
 #pragma unroll
         for (int f = 0; f < R; f++) {
             float v;
