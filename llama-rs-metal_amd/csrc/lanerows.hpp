@@ -174,7 +174,8 @@ struct LaneRows {
         static_assert(BITS == 4, "limb products take 4-bit codes");
 #pragma unroll
         for (int f = 0; f < R; f++) {
-            const float v = raw_to_f32<T>(sr[f]) * xl.dot4(c[f].w, cs[f]) + raw_to_f32<T>(br[f]) * xsum;
+            const float s = raw_to_f32<T>(sr[f]);
+            const float v = s * xl.dot4(c[f].w, cs[f]) + fmaf(8.0f, s, raw_to_f32<T>(br[f])) * xsum;
             res[f] = ok[f] ? v : 0.f;
         }
     }
@@ -188,31 +189,42 @@ struct LaneRows {
 // A lane's 32-element input chunk as six 4-bit limbs, for 4-bit codes on
 // the integer dot-product unit (v_dot8_u32_u4: eight code x limb products
 // per instruction, against one conversion and one FMA per code in
-// Chunk32::dot).  With 2^e > max|x| over the chunk, X_j = round(x_j 2^(22-e))
-// + 2^22 lies in [0, 2^23): the FMA x_j 2^(22-e) + 3 * 2^22 leaves it in the
-// float's mantissa bits (the exponent bit above them is 0 in [2^23, 2^24)).
-// W[l][i] holds nibble l of X_8i .. X_8i+7 in code order, so
+// Chunk32::dot).  With up just under 2^22 / max|x| over the chunk,
+// X_j = round(x_j up) + 2^22 lies in (0, 2^23): the FMA x_j up + 3 * 2^22
+// leaves it in the float's mantissa bits (the exponent bit above them is 0 in
+// [2^23, 2^24)).  W[l][i] holds nibble l of X_8i .. X_8i+7 in code order, so
 // sum_j c_j X_j = sum_l 16^l udot8(codes, W[l]) exactly; the 2^22 offset is
-// taken off with sum_j c_j.  One rounding of the exact integer sum
-// (2^-23 of the chunk maximum per input, the F32 FMA chain's order of
-// error).  A non-finite input makes the chunk's scale NaN.  Chunks whose
-// maximum lies below 2^-106 (subnormals included) take e = -105, so 2^(22-e)
-// stays finite and every X_j still fits: their error is 2^-128 per input.
+// taken off with sum_j c_j and the codes' centre with 8 sum_j X_j (an input's
+// rounding then weighs by the centred code).  One rounding of the exact integer
+// sum and one of each input, at most 2^-23 of the chunk maximum: a 128-expert
+// layer of 12 tokens is 3e-7 off its 64-bit result (uncentred, under a power of
+// two for `up`: 1.1e-6).  A non-finite input makes the chunk's scale NaN.
+// Chunks whose maximum lies below 2^-105 (subnormals included) are scaled as if
+// it were 2^-105, so `up` stays finite.
 struct XLimbs {
     uint32_t W[6][4];
-    float scale;  // 2^(e - 22)
+    int32_t clo, chi;  // 8 sum_j (X_j - 2^22) = clo + 4096 chi
+    float scale;       // 1 / up
     __device__ __forceinline__ void build(const float *x) {
         float m = 0.f;
 #pragma unroll
         for (int j = 0; j < 32; j++) m = fmaxf(m, fabsf(x[j]));
-        const int e = max(__builtin_amdgcn_frexp_expf(m), -105);
-        const float up = __builtin_amdgcn_ldexpf(1.0f, 22 - e);
-        scale = __builtin_isfinite(m) ? __builtin_amdgcn_ldexpf(1.0f, e - 22) : __builtin_nanf("");
+        // up = 4194300 / max and its inverse, each by way of numbers whose
+        // reciprocals are normal (the hardware's reciprocal, one ulp; one Newton
+        // step for 1 / up)
+        const float up4 = 262143.75f * __builtin_amdgcn_rcpf(0.25f * fmaxf(m, 0x1p-105f));  // up / 4
+        const float up = 4.0f * up4;
+        const float r0 = __builtin_amdgcn_rcpf(up4);
+        const float inv = 0.25f * fmaf(fmaf(-up4, r0, 1.0f), r0, r0);
+        scale = __builtin_isfinite(m) ? inv : __builtin_nanf("");
+        uint32_t sx = 0;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             uint32_t X[8];
 #pragma unroll
             for (int j = 0; j < 8; j++) X[j] = __float_as_uint(fmaf(x[8 * i + j], up, 12582912.0f));
+#pragma unroll
+            for (int j = 0; j < 8; j++) sx += X[j];
             // bytes k of the even (E) and odd (O) elements: E_k = (X0, X2, X4, X6) byte k
             uint32_t E[3], O[3];
 #pragma unroll
@@ -234,28 +246,33 @@ struct XLimbs {
                 W[2 * k + 1][i] = ((E[k] >> 4) & 0x0f0f0f0fu) | (O[k] & 0xf0f0f0f0u);
             }
         }
+        // the float bits are 0x4b000000 + X_j: 32 of them, and the offset, off
+        const int32_t c8 = (int32_t)(sx - 32u * 0x4b000000u - (32u << 22)) * 8;  // |.| <= 2^30
+        clo = c8 & 4095;
+        chi = c8 >> 12;
     }
-    // sum_j c_j of 32 4-bit codes (the offset term of dot4)
+    // the offset term of dot4 for a row's 32 4-bit codes: -2^10 sum_j c_j
     static __device__ __forceinline__ uint32_t code_sum4(const uint32_t *w) {
         uint32_t cs = 0;
 #pragma unroll
         for (int i = 0; i < 4; i++) cs = __builtin_amdgcn_udot8(w[i], 0x11111111u, cs, false);
-        return cs;
+        return 0u - (cs << 10);
     }
-    // sum_j c_j x_j for the chunk's 32 4-bit codes (4 words, code j of word i
-    // multiplies element 8i + j); cs = code_sum4(w)
+    // sum_j (c_j - 8) x_j for the chunk's 32 4-bit codes (4 words, code j of word i
+    // multiplies element 8i + j); cs = code_sum4(w).  The offset terms start the
+    // accumulators (modulo 2^32).
     __device__ __forceinline__ float dot4(const uint32_t *w, uint32_t cs) const {
         uint32_t P[6];
 #pragma unroll
         for (int l = 0; l < 6; l++) {
-            uint32_t acc = 0;
+            uint32_t acc = l == 0 ? 0u - (uint32_t)clo : l == 3 ? cs - (uint32_t)chi : 0u;
 #pragma unroll
             for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_udot8(w[i], W[l][i], acc, false);
-            P[l] = acc;  // <= 32 * 15 * 15
+            P[l] = acc;
         }
-        const uint32_t lo = P[0] + (P[1] << 4) + (P[2] << 8);                       // < 2^21
-        const int32_t hi = (int32_t)(P[3] + (P[4] << 4) + (P[5] << 8)) - (int32_t)(cs << 10);
-        return ((float)lo + (float)hi * 4096.0f) * scale;  // (sum c X - 2^22 sum c) 2^(e-22)
+        const int32_t lo = (int32_t)(P[0] + (P[1] << 4) + (P[2] << 8));  // |.| < 2^22
+        const int32_t hi = (int32_t)(P[3] + (P[4] << 4) + (P[5] << 8));
+        return ((float)lo + (float)hi * 4096.0f) * scale;  // sum (c - 8) (X - 2^22) / up
     }
 };
 
