@@ -66,7 +66,7 @@ struct Chunk32 {
     // F16 = true: eight codes at a time to centred f16 (codes16.hpp),
     // multiplied by mixed-precision FMAs: fewer instructions, for waves whose
     // arithmetic repeats over inputs (seg_down at 64 tokens 90 -> 68 us).
-    static constexpr int kRun = BITS == 8 ? 4 : 8;
+    static constexpr int kRun = BITS == 2 ? 8 : 4;
     static constexpr float kCentre = BITS ? (float)(1 << (BITS ? BITS - 1 : 0)) : 0.f;
     template <bool F16>
     __device__ __forceinline__ float dot(const float *x, [[maybe_unused]] const float *rs) const {
