@@ -74,7 +74,7 @@ moe_status moe_gpu_create(int device, moe_gpu **out) {
         hipEventCreateWithFlags(&g->ev_fork, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&g->ev_join, hipEventDisableTiming) != hipSuccess ||
         hipMalloc(reinterpret_cast<void **>(&g->arrive), 256) != hipSuccess ||
-        hipMemset(g->arrive, 0, 256) != hipSuccess) {
+        hipMemset(g->arrive, 0, 256) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
         if (g->arrive) (void)hipFree(g->arrive);
         delete g;
         return MOE_ERR_GPU;
@@ -131,7 +131,10 @@ moe_status moe_zeros(moe_gpu *g, uint64_t n, moe_buffer *out) {
     void *p = nullptr;
     st = alloc_bytes(g, n * 4, &p);
     if (st) return st;
+    // (the fill runs on the null stream, which the gpu's own streams do not
+    // wait for)
     hipError_t e = hipMemset(p, 0, n * 4);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) return gpu_err(g, e, "zero fill");
     *out = moe_buffer{p, n};
     return MOE_OK;
@@ -191,6 +194,7 @@ moe_status moe_clear(moe_gpu *g, moe_buffer b) {
     if ((st = check_own(g, {rng(b)}))) return st;
     hipError_t e = hipStreamSynchronize(g->stream);
     if (e == hipSuccess) e = hipMemset(b.ptr, 0, b.len * 4);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     return launched(g, e, "clear");
 }
 

@@ -328,6 +328,27 @@ def test_allocation_error_carries_bytes(gpu):
     gpu.release(b)
 
 
+def test_zero_fills_end_before_the_call_returns(gpu):
+    """A zero fill that queues behind a large one is over before a product
+    writes the buffer: the fills run on the null stream, which the gpu's own
+    streams do not wait for."""
+    w = synth.normal(61, 64 * 256)
+    x = synth.normal(62, 64)
+    wt, xb = gpu.weight_tensor(Tensor.dense([64, 256], w)), gpu.upload(x)
+    for clear in (False, True):
+        big = gpu.zeros(1 << 28)
+        y = gpu.zeros(256)
+        if clear:
+            gpu.clear(big)
+            gpu.clear(y)
+        with gpu.batch() as b:
+            b.matmul(wt, xb, y, 1)
+        close(gpu.read(y), w.reshape(256, 64) @ x)
+        gpu.release(big)
+        gpu.release(y)
+    gpu.release(xb)
+
+
 @pytest.mark.parametrize("n,heads,pad", [(1, 2, 0), (64, 5, 3), (128, 16, 0), (255, 2, 1), (260, 3, 4), (1023, 1, 0),
                                          (2047, 2, 0), (2048, 3, 0), (2052, 2, 0), (5000, 2, 8)])
 @pytest.mark.parametrize("dtype", [F32, F16, BF16])
