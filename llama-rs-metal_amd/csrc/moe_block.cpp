@@ -7,7 +7,8 @@
 //                     grouped expert products, one combine
 //   MOE_PATH_AUTO     fused 3-kernel decode for one token; bf16 MFMA for
 //                     prefill-sized segments; the batched decode
-//                     (k_batched.hip) for a few tokens; grouped otherwise
+//                     (k_batched.hip, k_split.hip) for shorter ones; grouped
+//                     otherwise
 #include "abi_common.hpp"
 
 namespace {
@@ -684,7 +685,9 @@ moe_status block_entry(moe_gpu *g, const moe_block_weights *w, moe_buffer x, moe
     }
     if (io->path == MOE_PATH_OPS)
         return run_ops(g, w, d, xin, xraw, o, T, io, L, ws, logits, ids, wts);
-    if (io->path == MOE_PATH_AUTO && batched_ok(w) && aligned16(xin) && aligned16(ws))
+    // (one grid row per run of pairs: at most 65535 of them)
+    if (io->path == MOE_PATH_AUTO && batched_ok(w) && aligned16(xin) && aligned16(ws) &&
+        seg_max_entries((uint32_t)(T * d.K), (uint32_t)d.E) <= 65535)
         return run_batched(g, w, d, xin, xraw, o, T, io, L, ws, logits, ids, wts);
     return run_grouped(g, w, d, xin, xraw, o, T, io, L, ws, logits, ids, wts);
 }

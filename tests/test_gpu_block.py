@@ -370,6 +370,24 @@ def test_batched_split_products(gpu, experts, ff, ffs, T):
     check_in_block_dispatch(bw, T, got[2], wsd["ws"], tm=bw.workspace_layout(T)["tile_pairs_batched"])
 
 
+def test_more_runs_than_a_grid_holds(gpu):
+    """65535 tokens of 9 experts each, h too short for the MFMA path and ff 384
+    (no power-of-two row): more runs of 8 pairs than one grid dimension holds,
+    so the grouped path takes the call.  The rows repeat every 61 tokens, and
+    so must every output; the first 61 are compared with the oracle."""
+    T, h, n = 65535, 64, 61
+    print(f"[case] runs beyond a grid T={T}", flush=True)
+    kinds = {"router": DENSE, "experts": (4, 32, BF16), "shared": (4, 32, BF16), "shared_gate": DENSE}
+    blk = HostBlock(h, 12, 9, 384, 0, kinds, seed=77, random_experts=True)
+    bw = blk.upload(gpu)
+    base = synth.normal(771, n * h).reshape(n, h)
+    got, prof = profiled(gpu, lambda: run_block(gpu, bw, np.resize(base, (T, h)), T, PATH_AUTO))
+    assert "seg_gateup" not in prof, sorted(prof)
+    check_against_oracle(blk, base, tuple(g[:n] for g in got))
+    out = got[0]
+    assert np.array_equal(out, np.resize(out[:n], out.shape))
+
+
 def test_route_dispatch_grids_in_sequence(gpu):
     """The fused route + dispatch launch counts its finished blocks on a
     device word that its last block puts back to zero: launches of 1, 18, 2
