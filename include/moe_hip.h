@@ -239,7 +239,7 @@ moe_status moe_pack_weight(moe_gpu *gpu, const moe_weight *w, moe_packed_weight 
 enum {
     MOE_PATH_AUTO = 0,   /* fused decode for one token; bf16 MFMA when the mean expert
                             segment holds >= 16 pairs; otherwise the batched decode
-                            (weight rows streamed once per run of 8 inputs) where the
+                            (weight rows streamed once per run of inputs) where the
                             shapes allow it, else VALU grouped */
     MOE_PATH_OPS = 1,     /* the reference's per-token op sequence (execute.rs:208-233) */
     MOE_PATH_GROUPED = 2, /* dispatch + grouped expert products on VALU (F32) */
