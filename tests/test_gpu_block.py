@@ -348,11 +348,11 @@ def test_batched_decode_layouts(gpu, experts, T):
 
 
 @pytest.mark.parametrize("experts", [(2, 32, BF16), (4, 64, F16), (4, 128, F32), (8, 32, BF16), (8, 128, F16)])
-@pytest.mark.parametrize("ff,ffs,T", [(128, 128, 30), (384, 0, 17), (384, 256, 100)])
+@pytest.mark.parametrize("ff,ffs,T", [(640, 0, 1), (640, 640, 2), (128, 128, 30), (384, 0, 17), (384, 256, 100)])
 def test_batched_split_products(gpu, experts, ff, ffs, T):
     """The batched decode where the expert segments are long enough for the
-    split products (and, with ff 384, where the VALU rows do not take the down
-    rows at any length): ragged segments of 0 to over 32 pairs, segments that
+    split products (and, with ff 384 and 640, where the VALU rows do not take the
+    down rows at any length, from one token on): ragged segments of 0 to over 32 pairs, segments that
     end inside and at a 16-pair entry, the shared expert on either side of its
     own threshold, every code width; and the router's F32 matrix-core product
     where it has enough logits."""
