@@ -237,7 +237,8 @@ __device__ __forceinline__ void put_chunk(Stage &st, int r, int c, const float *
 #pragma unroll
     for (int j = 0; j < 8; j++) sum += v[j];
     // (a NaN, which fmaxf drops, and an infinity reach the row's products as
-    // NaN: through hi, and through lo = inf - inf)
+    // NaN, through hi and through lo = inf - inf; body() computes such outputs
+    // again from decoded weights)
     sum += dpp_f<kDppQuad1>(sum);
     sum += dpp_f<kDppQuad2>(sum);
     // 2^e > m; clamped so that 2^(15-e) stays finite (rows below 2^-106 keep
@@ -257,6 +258,35 @@ __device__ __forceinline__ void put_chunk(Stage &st, int r, int c, const float *
     *reinterpret_cast<u32x4 *>(&st.a[1][r][at]) = lo;
     if ((c & 3) == 0) st.sums[c >> 2][r] = sum;
     if (c == 0) st.scale[r] = __builtin_amdgcn_ldexpf(1.0f, e - 15);
+}
+
+// One output in F32 with its weights decoded first (code * scale + bias, two
+// roundings, the values Tensor::decode produces), for results the split has no
+// finite value for: an infinite input has no lo term (inf - inf), and inputs
+// above about 2^114 can overflow a group's sum, whose scale is applied after it.
+// A lane's own loop over the row: such results are rare.
+template <int BITS, int T>
+__device__ __forceinline__ float decoded_dot(const WDesc &wd, uint64_t el, const float *x) {
+    constexpr int P = 32 / BITS;
+    const uint32_t *wp = reinterpret_cast<const uint32_t *>(wd.data) + el / P;
+    float acc = 0.f;
+#pragma unroll 1
+    for (uint32_t k = 0; k < wd.in; k += P) {
+        const uint64_t g = (el + k) >> wd.gshift;
+        const float s = raw_to_f32<T>(load_raw<T>(wd.scales, g)), b = raw_to_f32<T>(load_raw<T>(wd.biases, g));
+        float c[P];
+        unpack_word<BITS>(wp[k / P], c);
+#pragma unroll
+        for (int j = 0; j < P; j++) {
+            float w;
+            {
+#pragma clang fp contract(off)
+                w = c[j] * s + b;
+            }
+            acc = fmaf(w, x[k + j], acc);
+        }
+    }
+    return acc;
 }
 
 // Rows [beg, end) of the entry (at most kRows), weight rows of block column bx.
@@ -397,6 +427,7 @@ __device__ __forceinline__ void body(const Args &a, Stage *st, uint32_t bx, uint
         if (u + 3 < units) unit(u + 3, std::integral_constant<int, 3>{});
     }
     // acc[t][r]: input row 4 q + r, weight row 16 t + n16
+    uint32_t redo = 0;  // bit kOut * r + t: an output that is not finite
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const uint32_t p = beg + 4 * q + r;
@@ -406,13 +437,24 @@ __device__ __forceinline__ void body(const Args &a, Stage *st, uint32_t bx, uint
             const uint32_t c = col0 + 16 * t + n16;
             if (c >= out) continue;
             const uint64_t o = (uint64_t)p * out + c;
-            if constexpr (MODE == GATEUP) {
-                const float g = acc[t][r];
-                a.out[o] = g / (1.0f + expf(-g)) * acc[t + kOut][r];
-            } else {
-                a.out[o] = a.bias ? acc[t][r] + a.bias[o] : acc[t][r];
-            }
+            float v = acc[t][r];
+            if constexpr (MODE == GATEUP) v = v / (1.0f + expf(-v)) * acc[t + kOut][r];
+            else v = a.bias ? v + a.bias[o] : v;
+            if (!__builtin_isfinite(v)) redo |= 1u << (kOut * r + t);
+            a.out[o] = v;
         }
+    }
+    while (redo) {
+        const int i = __builtin_ctz(redo);
+        redo &= redo - 1;
+        const uint32_t p = beg + 4 * q + i / kOut, c = col0 + 16 * (i % kOut) + n16;
+        const uint64_t o = (uint64_t)p * out + c, row = ((uint64_t)e * out + c) * in;
+        const uint32_t src = MODE == GATEUP && a.perm ? a.perm[p] / a.k : p;
+        const float *x = a.in + (uint64_t)src * in;
+        float v = decoded_dot<BITS, T>(a.w, row, x);
+        if constexpr (MODE == GATEUP) v = v / (1.0f + expf(-v)) * decoded_dot<BITS, T>(a.w2, row, x);
+        else v = a.bias ? v + a.bias[o] : v;
+        a.out[o] = v;
     }
 }
 

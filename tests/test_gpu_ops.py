@@ -429,6 +429,38 @@ def test_matmul_split_nonfinite_rows(gpu):
         gpu.release(b_)
 
 
+@pytest.mark.parametrize("bits,group,st", [(2, 32, F32), (4, 64, BF16), (8, 128, F16)])
+@pytest.mark.parametrize("tokens", [4, 19])
+def test_matmul_split_infinities_and_overflow(gpu, bits, group, st, tokens):
+    """Tiled products of rows the split has no finite value for: every output
+    is the one its decoded weights give (oracle.matmul) -- an infinity of the
+    products' sign, NaN where two meet or a weight is 0 -- and finite inputs of
+    about 2^121, whose sums overflow before the group's scale, give finite results."""
+    print(f"[case] split infinities {bits}/{group}/{st} tokens={tokens}", flush=True)
+    n_in, out = 384, 70
+    q = synth.quantize_affine(synth.normal(41 + bits, n_in * out, 0.0, 2.0 ** -8), bits, group, st)
+    t = Tensor.affine([n_in, out], *q, bits, group, st)
+    x = synth.normal(42 + tokens, tokens * n_in).reshape(tokens, n_in)
+    x[0, 130] = np.inf
+    x[1, 383] = -np.inf
+    x[2, 5], x[2, 300] = np.inf, -np.inf
+    x[tokens - 1] *= np.float32(2.0 ** 121)
+    w, xb, y = gpu.weight_tensor(t), gpu.upload(x), gpu.zeros(tokens * out)
+    with gpu.batch() as b:
+        b.matmul(w, xb, y, tokens)
+    got = gpu.read(y).reshape(tokens, out)
+    ref = np.asarray(oracle.matmul(t, x, tokens)).reshape(tokens, out)
+    assert np.array_equal(got[:3], ref[:3], equal_nan=True)
+    assert np.isposinf(got[:2]).any() and np.isneginf(got[:2]).any()
+    # F32 sums of 384 products each: under 2^-20 of sum |w x|
+    wd = np.abs(np.asarray(oracle.decode(t), np.float64)).reshape(out, n_in)
+    mag = np.abs(x[3:].astype(np.float64)) @ wd.T
+    assert np.isfinite(ref[3:]).all() and np.isfinite(got[3:]).all()
+    assert np.all(np.abs(got[3:].astype(np.float64) - ref[3:]) <= 2.0 ** -20 * mag)
+    for b_ in (xb, y):
+        gpu.release(b_)
+
+
 def test_matmul_split_long_runs(gpu):
     """More token rows than one launch's grid holds (65535 entries of 16): the
     rows on both sides of the boundary and the last ones."""
