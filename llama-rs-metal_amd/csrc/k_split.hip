@@ -57,7 +57,7 @@ hipError_t launch_split_gateup(Prof *p, hipStream_t s, const char *name, const W
 
 hipError_t launch_split_rows(Prof *p, hipStream_t s, const char *name, const WDesc &w, const float *in,
                              const uint32_t *tiles, const uint32_t *ntiles, const uint32_t *offsets, uint32_t n,
-                             uint32_t entries, const float *bias, float *out) {
+                             uint32_t entries, float *out) {
     // Two tiles a wave halve the input staging per weight row; one while that
     // leaves the grid within two blocks a CU, where only the length of a block's
     // own chain counts (h 2048 -> 4096 rows at 32 / 128 / 1000 rows of input:
@@ -77,7 +77,6 @@ hipError_t launch_split_rows(Prof *p, hipStream_t s, const char *name, const WDe
         a.ntiles = ntiles;
         a.offsets = offsets;
         a.n = (uint32_t)(n - n0 < part ? n - n0 : part);
-        a.bias = bias ? bias + n0 * w.out : nullptr;
         a.out = out + n0 * w.out;
         e = split_dispatch(split::Launch{p, s, name, a, entries, nt}, split::ROWS);
     }

@@ -301,7 +301,7 @@ moe_status moe_matmul(moe_gpu *g, const moe_weight *w, moe_buffer x, moe_buffer 
     // cores 47 / 52 / 280, and a fifth of their error), the rest on the F32 ones
     if (tokens >= 4 && split_supported(d, (const float *)x.ptr))
         return launched(g, launch_split_rows(&g->prof, g->stream, "matmul_f32", d, (const float *)x.ptr, nullptr,
-                                             nullptr, nullptr, (uint32_t)tokens, 0, nullptr, (float *)y.ptr),
+                                             nullptr, nullptr, (uint32_t)tokens, 0, (float *)y.ptr),
                         "matmul");
     if (tokens >= 4 && f32mm_supported(d, (const float *)x.ptr))
         return launched(g, launch_f32mm(&g->prof, g->stream, "matmul_f32", d, (const float *)x.ptr,

@@ -284,15 +284,15 @@ moe_status run_batched(moe_gpu *g, const moe_block_weights *w, const Dims &d, co
     float *act = ws + L.act, *yexp = ws + L.yexp;
     const uint32_t entries = seg_max_entries(t32 * K, E);
     const float *bias = has(io->logit_bias) ? fp(io->logit_bias) : nullptr;
-    // Products over all tokens (router, shared expert) and over the dispatched
+    // Products of the shared expert over all tokens and of the dispatched
     // segments, each on VALU or as split products
-    auto rows = [&](hipStream_t st, const char *name, const WDesc &W, const float *in, bool segs, const float *b,
-                    float *o) {
+    auto rows = [&](hipStream_t st, const char *name, const WDesc &W, const float *in, bool segs, float *o) {
         const uint32_t n = segs ? t32 * K : t32;
         const bool split = split_ok(W) && (!seg_supported(W) || split_rows_better(W, n, segs ? E : 1));
         const uint32_t *tl = segs ? tiles : nullptr, *nt = segs ? ntiles : nullptr, *of = segs ? offsets : nullptr;
-        if (split) return launch_split_rows(p, st, name, W, in, tl, nt, of, n, entries, b, o);
-        return launch_seg_rows(p, st, name, W, in, tl, nt, of, segs ? 0 : n, segs ? entries : seg_max_entries(n, 0), b, o);
+        if (split) return launch_split_rows(p, st, name, W, in, tl, nt, of, n, entries, o);
+        return launch_seg_rows(p, st, name, W, in, tl, nt, of, segs ? 0 : n, segs ? entries : seg_max_entries(n, 0),
+                               nullptr, o);
     };
     auto gateup = [&](hipStream_t st, const char *name, const WDesc &G, const WDesc &U, bool segs, float *o) {
         const uint32_t n = segs ? t32 * K : t32;
@@ -313,23 +313,32 @@ moe_status run_batched(moe_gpu *g, const moe_block_weights *w, const Dims &d, co
     const float *so = nullptr, *sgv = nullptr;
     SideFork side{g, s};
     if (w->has_shared) TRY(side.mark());
-    // A router of many logits: the F32 matrix cores (K split over the grid, its
-    // partial sums in y16, which this path leaves idle), from 2^15 logits on:
-    // 512 dense rows at 64 / 500 tokens 9 / 21 us against 17 / 258 on VALU
+    // The router's product stays F32 (no split: the routing is exact given the
+    // logits, so they are the F32 product's).  A router of many logits: the F32
+    // matrix cores (K split over the grid, its partial sums in y16, which this
+    // path leaves idle), from 2^15 logits on: 512 dense rows at 64 / 500 tokens
+    // 9 / 21 us against 17 / 258 on VALU.  Fewer: VALU rows, or, for affine rows
+    // they do not take (no 2^k chunks), the per-token wave (1024 -> 256 4-bit
+    // rows at 2 / 33 tokens 3.7 / 4.6 us, on the F32 matrix cores 26)
     const WDesc R = wdesc(w->router);
     const bool f32_router = (uint64_t)t32 * E >= (1u << 15) && f32mm_supported(R, xin);
     const uint32_t rks = f32_router ? f32mm_ksplit(R, t32, (uint64_t)T * K * d.h / 2) : 1;
     float *parts = ws + L.y16;
     if (f32_router)
         TRY(launch_f32mm(p, s, "seg_router", R, xin, t32, rks, rks > 1 ? nullptr : bias, rks > 1 ? parts : logits));
-    else
-        TRY(rows(s, "seg_router", R, xin, false, bias, logits));
+    else if (seg_supported(R))
+        TRY(launch_seg_rows(p, s, "seg_router", R, xin, nullptr, nullptr, nullptr, t32, seg_max_entries(t32, 0), bias,
+                            logits));
+    else {
+        TRY(launch_gemv(p, s, R, xin, 0, nullptr, 1, logits, t32));
+        if (bias) TRY(launch_add(p, s, logits, bias, logits, T * d.E));
+    }
     if (w->has_shared) {
         float *sh = ws + L.sh_act, *sout = ws + L.sh_out, *sgt = ws + L.sh_gate;
         hipStream_t ss = g->side;
         TRY(side.enter());
         TRY(gateup(ss, "seg_shared_gateup", wdesc(w->shared_gate), wdesc(w->shared_up), false, sh));
-        TRY(rows(ss, "seg_shared_down", wdesc(w->shared_down), sh, false, nullptr, sout));
+        TRY(rows(ss, "seg_shared_down", wdesc(w->shared_down), sh, false, sout));
         TRY(launch_gemv(p, ss, gate_inp_desc(w->shared_gate_inp), xin, 0, nullptr, 1, sgt, t32));
         so = sout;
         sgv = sgt;
@@ -345,7 +354,7 @@ moe_status run_batched(moe_gpu *g, const moe_block_weights *w, const Dims &d, co
         TRY(launch_dispatch(p, s, ids, t32 * K, E, counts, offsets, perm, pos, seg_tokens(), tiles, ntiles));
     }
     TRY(gateup(s, "seg_gateup", wdesc(w->gate), wdesc(w->up), true, act));
-    TRY(rows(s, "seg_down", wdesc(w->down), act, true, nullptr, yexp));
+    TRY(rows(s, "seg_down", wdesc(w->down), act, true, yexp));
     TRY(side.join());
     TRY(launch_combine(p, s, yexp, pos, wts, K, so, sgv, io->residual ? xres : nullptr, out, t32,
                        (uint32_t)d.h));

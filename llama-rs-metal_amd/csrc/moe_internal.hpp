@@ -247,7 +247,7 @@ hipError_t launch_split_gateup(Prof *p, hipStream_t s, const char *name, const W
                                float *act);
 hipError_t launch_split_rows(Prof *p, hipStream_t s, const char *name, const WDesc &w, const float *in,
                              const uint32_t *tiles, const uint32_t *ntiles, const uint32_t *offsets, uint32_t n,
-                             uint32_t entries, const float *bias, float *out);
+                             uint32_t entries, float *out);
 // (expert, first position) of every run of `tm` pairs of the non-empty
 // segments, and their count (k_mfma.hip)
 hipError_t launch_tile_schedule(Prof *p, hipStream_t s, const uint32_t *offsets, uint32_t experts,

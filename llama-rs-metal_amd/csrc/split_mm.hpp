@@ -3,7 +3,7 @@
 //
 //   GATEUP  act[p, j] = silu(x_t . G_e[j]) * (x_t . U_e[j])   t = perm[p] / k
 //           (activation, crates/metal-backend/src/shaders/elementwise.metal:8-17)
-//   ROWS    out[p, r] = in_p . W_e[r] (+ bias[p, r])
+//   ROWS    out[p, r] = in_p . W_e[r]
 //           (Batch::matmul, crates/metal-backend/src/apple/ops/matrix.rs:63-148;
 //           expert_matmul(down), crates/model-runtime/src/execute.rs:225)
 //
@@ -75,7 +75,6 @@ struct Args {
     const uint32_t *ntiles;   // entry count (device), with tiles
     const uint32_t *offsets;  // segment bounds [e], [e + 1], with tiles
     uint32_t n;               // without tiles: input rows
-    const float *bias;        // ROWS: added to out[p, row] (or nullptr)
     float *out;               // [p, w.out]
 };
 
@@ -436,25 +435,22 @@ __device__ __forceinline__ void body(const Args &a, Stage *st, uint32_t bx, uint
         for (int t = 0; t < kOut; t++) {
             const uint32_t c = col0 + 16 * t + n16;
             if (c >= out) continue;
-            const uint64_t o = (uint64_t)p * out + c;
             float v = acc[t][r];
             if constexpr (MODE == GATEUP) v = v / (1.0f + expf(-v)) * acc[t + kOut][r];
-            else v = a.bias ? v + a.bias[o] : v;
             if (!__builtin_isfinite(v)) redo |= 1u << (kOut * r + t);
-            a.out[o] = v;
+            a.out[(uint64_t)p * out + c] = v;
         }
     }
     while (redo) {
         const int i = __builtin_ctz(redo);
         redo &= redo - 1;
         const uint32_t p = beg + 4 * q + i / kOut, c = col0 + 16 * (i % kOut) + n16;
-        const uint64_t o = (uint64_t)p * out + c, row = ((uint64_t)e * out + c) * in;
+        const uint64_t row = ((uint64_t)e * out + c) * in;
         const uint32_t src = MODE == GATEUP && a.perm ? a.perm[p] / a.k : p;
         const float *x = a.in + (uint64_t)src * in;
         float v = decoded_dot<BITS, T>(a.w, row, x);
         if constexpr (MODE == GATEUP) v = v / (1.0f + expf(-v)) * decoded_dot<BITS, T>(a.w2, row, x);
-        else v = a.bias ? v + a.bias[o] : v;
-        a.out[o] = v;
+        a.out[(uint64_t)p * out + c] = v;
     }
 }
 

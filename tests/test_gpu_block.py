@@ -370,6 +370,72 @@ def test_batched_split_products(gpu, experts, ff, ffs, T):
     check_in_block_dispatch(bw, T, got[2], wsd["ws"], tm=bw.workspace_layout(T)["tile_pairs_batched"])
 
 
+def outlier_router(h, E, seed):
+    """A 4-bit router whose rows hold one weight of exactly 0 in every 128
+    inputs (code 8 under scale s and bias -8 s), and the inputs' columns there."""
+    rng = np.random.default_rng(seed)
+    codes = rng.integers(0, 16, (E, h)).astype(np.uint32)
+    cols = np.arange(5, h, 128)
+    codes[:, cols] = 8
+    words = (codes.reshape(E, h // 8, 8) << (4 * np.arange(8, dtype=np.uint32))).sum(2, dtype=np.uint32)
+    n = E * h // 64
+    s = synth.f32_to_bf16_bits(np.full(n, 2.0 ** -7, np.float32))
+    b = synth.f32_to_bf16_bits(np.full(n, -(2.0 ** -4), np.float32))
+    return Tensor.affine([h, E], words.ravel(), s, b, 4, 64, BF16), cols
+
+
+@pytest.mark.parametrize("E,T", [(48, 100), (48, 190), (128, 200)])
+def test_batched_affine_router_is_f32(gpu, E, T):
+    """The batched path's affine router over inputs with a value of 2^30 in
+    every 128, at weights of exactly 0: F32 products do not see it, f16 terms
+    scaled to it would keep 10 bits of the other inputs.  Few enough logits for
+    the VALU rows, 96 tokens and more."""
+    print(f"[case] affine router E={E} T={T}", flush=True)
+    h = 256
+    kinds = {"router": DENSE, "experts": (4, 64, BF16)}
+    blk = HostBlock(h, E, 4, 128, 0, kinds, seed=95, random_experts=True)
+    blk.router, cols = outlier_router(h, E, 96)
+    x = synth.normal(4900 + T, T * h).reshape(T, h)
+    x[:, cols] *= np.float32(2.0 ** 30)
+    got = run_block(gpu, blk.upload(gpu), x, T, PATH_AUTO)
+    check_all_ids(blk, got)
+    assert rel_max_err(got[1], oracle.matmul(blk.router, x, T).reshape(T, E)) < 2e-6
+
+
+@pytest.mark.parametrize("h,T,kind", [(640, 2, (8, 64, BF16)), (640, 100, (4, 32, F32)), (384, 33, (2, 128, F16))])
+def test_batched_router_of_odd_rows_is_f32(gpu, h, T, kind):
+    """An affine router whose rows the VALU lanes do not take (h no 2^k
+    chunks): the per-token F32 wave, with the logit bias added."""
+    print(f"[case] odd router h={h} T={T} kind={kind}", flush=True)
+    kinds = {"router": kind, "experts": (4, 64, BF16)}
+    blk = HostBlock(h, 48, 4, 128, 0, kinds, seed=97 + T, random_experts=True)
+    x = synth.normal(4950 + T, T * h).reshape(T, h)
+    bias = hot_bias(T, 48, seed=T, frac=0.5, hot=5, boost=4.0)
+    got, prof = profiled(gpu, lambda: run_block(gpu, blk.upload(gpu), x, T, PATH_AUTO, bias=bias))
+    assert "gemv_generic" in prof and "seg_gateup" in prof and "seg_router" not in prof, sorted(prof)
+    check_all_ids(blk, got)
+    check_against_oracle(blk, x, got, bias=bias)
+
+
+@pytest.mark.parametrize("kind,T", [((4, 64, BF16), 128), ((8, 64, BF16), 128), (DENSE, 128), ((4, 64, BF16), 255)])
+def test_batched_routing_matches_oracle_f32_logits(gpu, kind, T):
+    """The batched path's ids against the oracle's routing of its own F32
+    logits: equal for every token whose K-th and K+1-th logits are further
+    apart than two F32 sums of h products may differ (h 2^-24 of the largest)."""
+    h, E, K = 2048, 128, 8
+    print(f"[case] routing vs oracle logits {kind} T={T}", flush=True)
+    blk = HostBlock(h, E, K, 128, 0, {"router": kind, "experts": (4, 64, BF16)}, seed=99, random_experts=True)
+    x = synth.normal(4990 + T, T * h).reshape(T, h)
+    got = run_block(gpu, blk.upload(gpu), x, T, PATH_AUTO)
+    ref = oracle.matmul(blk.router, x, T).reshape(T, E)
+    ids = oracle.route_tokens(ref, K, True)[0].reshape(T, K)
+    top = -np.sort(-ref, 1)
+    gaps = (top[:, :K] - top[:, 1:K + 1]).min(1)  # of the order among the selected too
+    clear = gaps > h * 2.0 ** -24 * np.abs(ref).max()
+    assert clear.sum() > T // 2
+    assert np.array_equal(got[2][clear], ids[clear])
+
+
 def test_more_runs_than_a_grid_holds(gpu):
     """65535 tokens of 9 experts each, h too short for the MFMA path and ff 384
     (no power-of-two row): more runs of 8 pairs than one grid dimension holds,
