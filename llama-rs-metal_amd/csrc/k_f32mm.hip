@@ -115,8 +115,14 @@ __device__ __forceinline__ void decode_w(const WRaw<BITS, T> &o, int j, float *v
     }
 }
 
-template <int BITS, int T, bool GATE>
-__global__ __launch_bounds__(kThreads) void f32mm_kernel(WDesc r, const float *__restrict__ x,
+// CH: independent sums the products of a tile's K range go to in turn, added
+// pairwise at the end.  A single sum rounds once per product, so its error
+// grows with the range; dense rows of the batched router take eight over ranges
+// of at most 256 values (f32mm_ranges), which the wave sums of the VALU rows
+// match (two waves per SIMD, which their registers would just miss, are what the
+// grid fills).
+template <int BITS, int T, bool GATE, int CH>
+__global__ __launch_bounds__(kThreads, CH == 8 ? 2 : 1) void f32mm_kernel(WDesc r, const float *__restrict__ x,
                                                               uint32_t tokens, uint32_t ksplit,
                                                               const float *__restrict__ bias,
                                                               float *__restrict__ out,
@@ -138,7 +144,7 @@ __global__ __launch_bounds__(kThreads) void f32mm_kernel(WDesc r, const float *_
     // weights: lane (i, hf) holds values 32hf .. 32hf + 31 of the iteration of
     // expert e0 + i (clamped; rows past E are never stored)
     const uint64_t wel = (uint64_t)min(e0 + i, E - 1) * h + kbeg + 32 * hf;
-    f32x16 acc = {};
+    f32x16 acc[CH] = {};
     f32x4 xr[2][2];  // native vectors: HIP's float4 struct would stay in scratch
     WRaw<BITS, T> wr[2];
     // shared-gate row (GATE): the block's K range of it goes to LDS once
@@ -194,7 +200,8 @@ __global__ __launch_bounds__(kThreads) void f32mm_kernel(WDesc r, const float *_
                 const f32x4 xv = *reinterpret_cast<const f32x4 *>(xrow + 16 * j + 4 * v);
 #pragma unroll
                 for (int c = 0; c < 4; c++)
-                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[c], wv16[4 * v + c], acc, 0, 0, 0);
+                    acc[(4 * v + c) % CH] =
+                        __builtin_amdgcn_mfma_f32_32x32x2f32(xv[c], wv16[4 * v + c], acc[(4 * v + c) % CH], 0, 0, 0);
             }
         }
     };
@@ -234,7 +241,13 @@ __global__ __launch_bounds__(kThreads) void f32mm_kernel(WDesc r, const float *_
         gsum += __shfl_xor(gsum, 4, 64);
         if (sch == 0 && t0 + srow < tokens) gout[((uint64_t)kr * gridDim.y + blockIdx.y) * tokens + t0 + srow] = gsum;
     }
-    // acc[q] = C[8(q/4) + 4(lane/32) + (q%4)][lane%32]: token row, expert column
+#pragma unroll
+    for (int w = 1; w < CH; w *= 2)
+#pragma unroll
+        for (int n = 0; n < CH; n += 2 * w)
+#pragma unroll
+            for (int q = 0; q < 16; q++) acc[n][q] += acc[n + w][q];
+    // acc[0][q] = C[8(q/4) + 4(lane/32) + (q%4)][lane%32]: token row, expert column
     const uint32_t e = e0 + i;
     if (e >= E) return;
 #pragma unroll
@@ -243,9 +256,9 @@ __global__ __launch_bounds__(kThreads) void f32mm_kernel(WDesc r, const float *_
         if (t >= tokens) continue;
         const uint64_t o = (uint64_t)t * E + e;
         if (ksplit == 1)
-            out[o] = bias ? acc[q] + bias[o] : acc[q];
+            out[o] = bias ? acc[0][q] + bias[o] : acc[0][q];
         else
-            out[(uint64_t)kr * tokens * E + o] = acc[q];
+            out[(uint64_t)kr * tokens * E + o] = acc[0][q];
     }
 }
 
@@ -261,13 +274,18 @@ struct Launch {
     uint16_t *xb16;
     const float *grow;
     float *gout;
+    int chains;
     template <int BITS, int T>
     hipError_t operator()() {
+        if (grow) return go<BITS, T, true, 1>();
+        if constexpr (BITS == 0)
+            if (chains == 8) return go<BITS, T, false, 8>();
+        return go<BITS, T, false, 1>();
+    }
+    template <int BITS, int T, bool GATE, int CH>
+    hipError_t go() {
         const dim3 grid((tokens + 31) / 32, (r.out + 32 * kWaves - 1) / (32 * kWaves), ksplit);
-        if (grow)
-            return launch_kernel(p, name, f32mm_kernel<BITS, T, true>, grid, dim3(kThreads), 0, s, r, x, tokens,
-                                 ksplit, bias, out, xb16, grow, gout);
-        return launch_kernel(p, name, f32mm_kernel<BITS, T, false>, grid, dim3(kThreads), 0, s, r, x, tokens,
+        return launch_kernel(p, name, f32mm_kernel<BITS, T, GATE, CH>, grid, dim3(kThreads), 0, s, r, x, tokens,
                              ksplit, bias, out, xb16, grow, gout);
     }
 };
@@ -298,13 +316,24 @@ uint32_t f32mm_ksplit(const WDesc &r, uint32_t tokens, uint64_t part_floats) {
     return ks;
 }
 
+// K ranges of the batched path's router: no longer than 256 values, so that its
+// logits are no further from the 64-bit ones than those of the VALU rows it
+// replaces (h 2048, 512 rows: dense 1.23e-7 on VALU, here in one sum over 256
+// values 2.9e-7, in eight 1.23e-7; affine 3.2e-7 on VALU with uncentred codes,
+// here 2.9e-7).  0: their partial sums do not fit.
+uint32_t f32mm_ranges(const WDesc &r, uint32_t tokens, uint64_t part_floats) {
+    uint32_t ks = f32mm_ksplit(r, tokens, part_floats);
+    if (r.in / ks > 256) ks = r.in % 256 == 0 ? r.in / 256 : r.in / 128;
+    return ks == 1 || (uint64_t)ks * tokens * r.out <= part_floats ? ks : 0;
+}
+
 hipError_t launch_f32mm(Prof *p, hipStream_t s, const char *name, const WDesc &r, const float *x,
                         uint32_t tokens, uint32_t ksplit, const float *bias, float *out, uint16_t *xb16,
-                        const float *grow, float *gout) {
+                        const float *grow, float *gout, int chains) {
     if (tokens == 0 || ksplit == 0 || r.in % (ksplit * 2 * f32mm::kIter)) return hipErrorInvalidValue;
     if (grow && (!gout || (reinterpret_cast<uintptr_t>(grow) & 15u) || r.in / ksplit > f32mm::kGateMax))
         return hipErrorInvalidValue;
-    return dispatch_kind(r, f32mm::Launch{p, s, name, r, x, tokens, ksplit, bias, out, xb16, grow, gout});
+    return dispatch_kind(r, f32mm::Launch{p, s, name, r, x, tokens, ksplit, bias, out, xb16, grow, gout, chains});
 }
 
 }  // namespace moehip

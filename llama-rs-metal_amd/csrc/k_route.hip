@@ -55,9 +55,16 @@ __global__ __launch_bounds__(64) void route_sum_kernel(const float *__restrict__
 #pragma unroll
             for (uint32_t i = 0; i < kSumParts; i++)  // ranges past the last repeat it, unused
                 p[i] = *reinterpret_cast<const V *>(parts + min(s0 + i, nsplit - 1) * stride + row + j);
+            // absent ranges count 0; pairs first (a chain of 16 would round more than
+            // the ranges' own sums do)
 #pragma unroll
             for (uint32_t i = 0; i < kSumParts; i++)
-                if (s0 + i < nsplit) v = s0 + i ? v + p[i] : p[i];
+                if (s0 + i >= nsplit) p[i] = V{};
+#pragma unroll
+            for (uint32_t w = 1; w < kSumParts; w *= 2)
+#pragma unroll
+                for (uint32_t i = 0; i < kSumParts; i += 2 * w) p[i] += p[i + w];
+            v += p[0];
         }
         if (bias) v += *reinterpret_cast<const V *>(bias + row + j);
         *reinterpret_cast<V *>(logits + row + j) = v;

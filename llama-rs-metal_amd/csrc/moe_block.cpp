@@ -317,15 +317,16 @@ moe_status run_batched(moe_gpu *g, const moe_block_weights *w, const Dims &d, co
     // logits, so they are the F32 product's).  A router of many logits: the F32
     // matrix cores (K split over the grid, its partial sums in y16, which this
     // path leaves idle), from 2^15 logits on: 512 dense rows at 64 / 500 tokens
-    // 9 / 21 us against 17 / 258 on VALU.  Fewer: VALU rows, or, for affine rows
+    // 12 / 22 us against 32 / 239 on VALU.  Fewer: VALU rows, or, for affine rows
     // they do not take (no 2^k chunks), the per-token wave (1024 -> 256 4-bit
     // rows at 2 / 33 tokens 3.7 / 4.6 us, on the F32 matrix cores 26)
     const WDesc R = wdesc(w->router);
-    const bool f32_router = (uint64_t)t32 * E >= (1u << 15) && f32mm_supported(R, xin);
-    const uint32_t rks = f32_router ? f32mm_ksplit(R, t32, (uint64_t)T * K * d.h / 2) : 1;
+    uint32_t rks = 0;
+    if ((uint64_t)t32 * E >= (1u << 15) && f32mm_supported(R, xin)) rks = f32mm_ranges(R, t32, (uint64_t)T * K * d.h / 2);
     float *parts = ws + L.y16;
-    if (f32_router)
-        TRY(launch_f32mm(p, s, "seg_router", R, xin, t32, rks, rks > 1 ? nullptr : bias, rks > 1 ? parts : logits));
+    if (rks)
+        TRY(launch_f32mm(p, s, "seg_router", R, xin, t32, rks, rks > 1 ? nullptr : bias, rks > 1 ? parts : logits,
+                         nullptr, nullptr, nullptr, R.bits ? 1 : 8));
     else if (seg_supported(R))
         TRY(launch_seg_rows(p, s, "seg_router", R, xin, nullptr, nullptr, nullptr, t32, seg_max_entries(t32, 0), bias,
                             logits));

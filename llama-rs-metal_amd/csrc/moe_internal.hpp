@@ -93,6 +93,9 @@ hipError_t launch_route_sum(Prof *p, hipStream_t s, const float *parts, uint32_t
 // router's).  Profiled under `name`.
 bool f32mm_supported(const WDesc &w, const float *x);
 uint32_t f32mm_ksplit(const WDesc &w, uint32_t tokens, uint64_t part_floats);
+// The K ranges of the batched path's router (0: their partial sums do not fit);
+// dense rows are to be launched with eight `chains` (independent sums).
+uint32_t f32mm_ranges(const WDesc &w, uint32_t tokens, uint64_t part_floats);
 // xb16 (optional, [tokens, in]): x rounded to bf16, written on the way.
 // grow: a dense F32 row (16-byte aligned) whose product with every token's x
 // the router also forms, one partial sum per K range and column of 128
@@ -102,7 +105,8 @@ uint32_t f32mm_gate_max();
 uint32_t f32mm_columns(const WDesc &w);
 hipError_t launch_f32mm(Prof *p, hipStream_t s, const char *name, const WDesc &w, const float *x,
                         uint32_t tokens, uint32_t ksplit, const float *bias, float *out,
-                        uint16_t *xb16 = nullptr, const float *grow = nullptr, float *gout = nullptr);
+                        uint16_t *xb16 = nullptr, const float *grow = nullptr, float *gout = nullptr,
+                        int chains = 1);
 hipError_t launch_route(Prof *p, hipStream_t s, const float *logits, uint32_t experts, uint32_t k,
                         int normalize, uint32_t tokens, uint32_t *ids, float *weights);
 // With `tiles` it also writes the work list of tm-pair runs that

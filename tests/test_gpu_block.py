@@ -436,6 +436,23 @@ def test_batched_routing_matches_oracle_f32_logits(gpu, kind, T):
     assert np.array_equal(got[2][clear], ids[clear])
 
 
+@pytest.mark.parametrize("kind,K,T", [(DENSE, 10, 64), (DENSE, 10, 500), (("dense", BF16), 10, 130), (DENSE, 1, 64)])
+def test_batched_dense_router_sums(gpu, kind, K, T):
+    """The batched path's dense router logits of 512 rows of 2048 against 64
+    bits: on the F32 matrix cores as near as a VALU lane's sum of 32 products
+    (an F32 sum of n products of random sign rounds to 2^-24 / sqrt(3) of it
+    times sqrt(n / 2)), also where the K ranges' partial sums do not fit (K 1)."""
+    h, E = 2048, 512
+    print(f"[case] dense router sums {kind} K={K} T={T}", flush=True)
+    blk = HostBlock(h, E, K, 128, 0, {"router": kind, "experts": (4, 64, BF16)}, seed=88, random_experts=True)
+    x = synth.normal(4970 + T, T * h).reshape(T, h)
+    got = run_block(gpu, blk.upload(gpu), x, T, PATH_AUTO)
+    check_all_ids(blk, got)
+    ref = x.astype(np.float64) @ np.asarray(oracle.decode(blk.router), np.float64).reshape(E, h).T
+    err = np.linalg.norm(got[1] - ref) / np.linalg.norm(ref)
+    assert err <= 2.0 ** -24 / np.sqrt(3) * np.sqrt(32 / 2), err
+
+
 def test_more_runs_than_a_grid_holds(gpu):
     """65535 tokens of 9 experts each, h too short for the MFMA path and ff 384
     (no power-of-two row): more runs of 8 pairs than one grid dimension holds,
