@@ -77,7 +77,7 @@ __global__ __launch_bounds__(kNormThreads) void norm_kernel(const float *__restr
         } else {
 #pragma unroll
             for (uint32_t j = 0; j < 4; j++)
-                if (i + j < n) v[j] = xr[i + j];
+                if ((uint64_t)i + j < n) v[j] = xr[i + j];
         }
         return v;
     };
@@ -89,8 +89,9 @@ __global__ __launch_bounds__(kNormThreads) void norm_kernel(const float *__restr
     for (uint32_t q = 0; q < kNormHold; q++)
 #pragma unroll
         for (int j = 0; j < 4; j++) s += hold[q][j] * hold[q][j];
-    for (uint32_t i = 4 * tid + kNormHold * step; i < n; i += step) {
-        const f32x4e v = load4(i);
+    // (64-bit: i + step may pass 2^32 for the longest rows)
+    for (uint64_t i = 4 * tid + kNormHold * step; i < n; i += step) {
+        const f32x4e v = load4((uint32_t)i);
 #pragma unroll
         for (int j = 0; j < 4; j++) s += v[j] * v[j];
     }
@@ -110,12 +111,12 @@ __global__ __launch_bounds__(kNormThreads) void norm_kernel(const float *__restr
         } else {
 #pragma unroll
             for (uint32_t j = 0; j < 4; j++)
-                if (i + j < n) yr[i + j] = v[j] * inv * load_scalar<T>(w, i + j);
+                if ((uint64_t)i + j < n) yr[i + j] = v[j] * inv * load_scalar<T>(w, i + j);
         }
     };
 #pragma unroll
     for (uint32_t q = 0; q < kNormHold; q++) store4(4 * tid + q * step, hold[q]);
-    for (uint32_t i = 4 * tid + kNormHold * step; i < n; i += step) store4(i, load4(i));
+    for (uint64_t i = 4 * tid + kNormHold * step; i < n; i += step) store4((uint32_t)i, load4((uint32_t)i));
 }
 
 // out[t, i] = sum_k w[t,k] * yexp[pos[t*K+k]*h + i]          (mix, k ascending)
@@ -168,7 +169,7 @@ hipError_t launch_norm(Prof *p, hipStream_t s, const float *x, const void *w, ui
     auto kern = vec ? (wtype == 0 ? norm_kernel<0, true> : wtype == 1 ? norm_kernel<1, true> : norm_kernel<30, true>)
                     : (wtype == 0 ? norm_kernel<0, false> : wtype == 1 ? norm_kernel<1, false> : norm_kernel<30, false>);
     // short rows (attention heads) keep one wave: four values a lane
-    const uint32_t groups = (n + 3) / 4;
+    const uint32_t groups = n / 4 + (n % 4 != 0);
     const uint32_t threads = groups < kNormThreads ? (groups + 63) / 64 * 64 : kNormThreads;
     return launch_kernel(p, "norm", kern, dim3(heads), dim3(threads), 0, s, x, w, y, n, stride, eps);
 }

@@ -382,6 +382,33 @@ def test_norm_rows(gpu, n, heads, pad, dtype):
     gpu.release(buf)
 
 
+def test_norm_longest_rows(gpu):
+    """One row whose length lies within a block's stride of 2^32 (17 GB): the
+    walk over it ends, and its first and last values are normalised."""
+    from hip_backend.api import MoeRegionC, MoeWeightC, Weight
+    n = (1 << 32) - 512
+    print(f"[case] norm n={n}", flush=True)
+    x, y, wb = gpu.zeros(n), gpu.zeros(n), gpu.zeros(n // 2)
+    w = MoeWeightC()
+    w.data = MoeRegionC()
+    w.data.ptr, w.data.bytes = wb.ptr, 2 * n
+    w.dtype, w.ndims, w.dims[0] = BF16, 1, n
+    first, last = np.array([3.0, -1.0], np.float32), np.array([2.0, 4.0], np.float32)
+    for b_, at, v in ((x, 0, first), (x, n - 2, last)):
+        gpu.write(b_.view(at, 2), v)
+    one = synth.f32_to_bf16_bits(np.array([1.0, 0.5], np.float32)).view(np.float32)
+    for at in (0, n // 2 - 1):
+        gpu.write(wb.view(at, 1), one)
+    with gpu.batch() as b:
+        b.norm(x, Weight(w, [w.data], [n], 0), y, 1, n, 1e-5)
+    scale = np.array([1.0, 0.5]) / np.sqrt((9.0 + 1 + 4 + 16) / n + 1e-5)
+    np.testing.assert_allclose(gpu.read(y.view(0, 2)), first * scale, rtol=1e-6)
+    np.testing.assert_allclose(gpu.read(y.view(n - 2, 2)), last * scale, rtol=1e-6)
+    assert not gpu.read(y.view(2, 4096)).any() and not gpu.read(y.view(n - 4098, 4096)).any()
+    for b_ in (x, y, wb):
+        gpu.release(b_)
+
+
 @pytest.mark.parametrize("bits,group,st", [(2, 32, F32), (2, 64, BF16), (2, 128, F16), (4, 32, BF16), (4, 64, F16),
                                            (4, 128, F32), (8, 32, F16), (8, 64, F32), (8, 128, BF16)])
 @pytest.mark.parametrize("n_in,out,tokens", [(128, 1, 4), (256, 17, 15), (384, 130, 16), (512, 64, 17), (640, 255, 33),
