@@ -52,6 +52,13 @@ void prof_collect(Prof *p, hipStream_t s) {
 
 }  // namespace moehip
 
+// Zeroes memory that nothing else uses yet, on the gpu's own stream: the fill is
+// over before any batch, and waits for no work of the host's on other streams.
+static hipError_t zero_new(moe_gpu *g, void *p, uint64_t bytes) {
+    const hipError_t e = hipMemsetAsync(p, 0, bytes, g->stream);
+    return e == hipSuccess ? hipStreamSynchronize(g->stream) : e;
+}
+
 // ================================================================= device ==
 extern "C" {
 
@@ -74,7 +81,7 @@ moe_status moe_gpu_create(int device, moe_gpu **out) {
         hipEventCreateWithFlags(&g->ev_fork, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&g->ev_join, hipEventDisableTiming) != hipSuccess ||
         hipMalloc(reinterpret_cast<void **>(&g->arrive), 256) != hipSuccess ||
-        hipMemset(g->arrive, 0, 256) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
+        zero_new(g, g->arrive, 256) != hipSuccess) {
         if (g->arrive) (void)hipFree(g->arrive);
         delete g;
         return MOE_ERR_GPU;
@@ -131,10 +138,7 @@ moe_status moe_zeros(moe_gpu *g, uint64_t n, moe_buffer *out) {
     void *p = nullptr;
     st = alloc_bytes(g, n * 4, &p);
     if (st) return st;
-    // (the fill runs on the null stream, which the gpu's own streams do not
-    // wait for)
-    hipError_t e = hipMemset(p, 0, n * 4);
-    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    hipError_t e = zero_new(g, p, n * 4);
     if (e != hipSuccess) return gpu_err(g, e, "zero fill");
     *out = moe_buffer{p, n};
     return MOE_OK;
@@ -192,6 +196,9 @@ moe_status moe_clear(moe_gpu *g, moe_buffer b) {
     moe_status st = need_no_batch(g);
     if (st) return st;
     if ((st = check_own(g, {rng(b)}))) return st;
+    // (like read and write, behind the null stream's work, which may still use
+    // registered memory; the gpu's own streams do not wait for that stream, so
+    // the fill ends first)
     hipError_t e = hipStreamSynchronize(g->stream);
     if (e == hipSuccess) e = hipMemset(b.ptr, 0, b.len * 4);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);

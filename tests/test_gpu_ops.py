@@ -349,6 +349,27 @@ def test_zero_fills_end_before_the_call_returns(gpu):
     gpu.release(xb)
 
 
+def test_zeros_wait_for_no_other_stream(gpu):
+    """moe_zeros returns while a host's own work on the null stream still runs
+    (about 0.1 s of fills of 8 GB, queued through the HIP runtime in use)."""
+    import ctypes
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    hip = ctypes.CDLL(path)
+    hip.hipMemsetD32Async.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t, ctypes.c_void_p]
+    hip.hipStreamQuery.argtypes = hip.hipStreamSynchronize.argtypes = [ctypes.c_void_p]
+    big = gpu.zeros(1 << 31)
+    for _ in range(50):
+        assert hip.hipMemsetD32Async(big.ptr, 1, 1 << 31, None) == 0
+    small = gpu.zeros(1000)
+    busy = hip.hipStreamQuery(None)
+    assert hip.hipStreamSynchronize(None) == 0
+    assert busy == 600  # hipErrorNotReady
+    assert not gpu.read(small).any()
+    for b_ in (big, small):
+        gpu.release(b_)
+
+
 @pytest.mark.parametrize("n,heads,pad", [(1, 2, 0), (64, 5, 3), (128, 16, 0), (255, 2, 1), (260, 3, 4), (1023, 1, 0),
                                          (2047, 2, 0), (2048, 3, 0), (2052, 2, 0), (5000, 2, 8)])
 @pytest.mark.parametrize("dtype", [F32, F16, BF16])
