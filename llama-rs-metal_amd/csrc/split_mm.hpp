@@ -14,7 +14,8 @@
 // 2^-24 of it off on average.  So sum(code * x) over a quantization group is
 // two matrix products whose products are exact in the F32 accumulator, and the
 // group's scale and bias are applied to that sum in F32:
-//   out = sum_g scale_g * D_g + (bias_g + 2^(bits-1) scale_g) * sum_g(x).
+//   out = sum_g scale_g * D_g + (bias_g + 2^(bits-1) scale_g) * sum_g(x),
+// a group's two terms first, so that the running sum rounds once per group.
 // The centred codes and the one F32 addition per group leave it closer to the
 // 64-bit product than a chain of F32 multiply-adds over the unsigned codes.
 //
@@ -25,7 +26,8 @@
 // gate/up 615 us on VALU, 196 here (3.1 TB/s of codes; without the products 157),
 // down 411 -> 114.  h 2048 -> 4096 rows over 2000 tokens 144 us (233 TFLOP/s as
 // F32), where the F32 matrix cores take 280.  Against 64 bits the products of
-// 700 rows are off by 1.7e-7, those of the F32 matrix cores by 8.1e-7.
+// 2048 values in groups of 64 are off by 1.4e-7, those of the F32 matrix cores
+// by 8.1e-7.
 // Entries of 32 and 64 rows, four tiles a wave, eight waves a block and codes
 // four units ahead were all slower (fewer waves per SIMD; 26 to 60%).
 //
@@ -81,7 +83,7 @@ struct Args {
 // One buffer of the block's input rows for one unit.
 struct Stage {
     uint8_t a[2][kRows][kUnit * 2];  // hi and lo terms, f16
-    float sums[4][kRows];            // sums of x over 32 values, per group of 32
+    float sums[4][kRows];            // sums of the scaled x over 32 values, per group of 32
     float scale[kRows];              // 2^(e-15): a * scale = x
 };
 
@@ -255,14 +257,14 @@ __device__ __forceinline__ void put_chunk(Stage &st, int r, int c, const float *
     const int at = 16 * (c ^ (r & 15));
     *reinterpret_cast<u32x4 *>(&st.a[0][r][at]) = hi;
     *reinterpret_cast<u32x4 *>(&st.a[1][r][at]) = lo;
-    if ((c & 3) == 0) st.sums[c >> 2][r] = sum;
+    if ((c & 3) == 0) st.sums[c >> 2][r] = sum * up;
     if (c == 0) st.scale[r] = __builtin_amdgcn_ldexpf(1.0f, e - 15);
 }
 
 // One output in F32 with its weights decoded first (code * scale + bias, two
 // roundings, the values Tensor::decode produces), for results the split has no
 // finite value for: an infinite input has no lo term (inf - inf), and inputs
-// above about 2^114 can overflow a group's sum, whose scale is applied after it.
+// above about 2^122 can overflow the sum of a group's inputs.
 // A lane's own loop over the row: such results are rare.
 template <int BITS, int T>
 __device__ __forceinline__ float decoded_dot(const WDesc &wd, uint64_t el, const float *x) {
@@ -371,7 +373,7 @@ __device__ __forceinline__ void body(const Args &a, Stage *st, uint32_t bx, uint
                     d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, c, d[t], 0, 0, 0);
                 }
             }
-            // sums of the rows' x over the group
+            // sums of the rows' scaled x over the group
             f32x4 xs = *reinterpret_cast<const f32x4 *>(&cur.sums[g * FG][4 * q]);
 #pragma unroll
             for (int f = 1; f < FG; f++) {
@@ -384,7 +386,7 @@ __device__ __forceinline__ void body(const Args &a, Stage *st, uint32_t bx, uint
                 const float s = Scales<T, GS>::value(sw[t][0], g);
                 const float b = fmaf((float)(1 << (BITS - 1)), s, Scales<T, GS>::value(sw[t][1], g));
 #pragma unroll
-                for (int r = 0; r < 4; r++) acc[t][r] = fmaf(b, xs[r], fmaf(s, d[t][r] * fx[r], acc[t][r]));
+                for (int r = 0; r < 4; r++) acc[t][r] = fmaf(fmaf(b, xs[r], s * d[t][r]), fx[r], acc[t][r]);
                 // the group's sums are added here: left to itself the compiler
                 // sinks every group's additions below the last one's products,
                 // holding all their sums (half as many waves fit)

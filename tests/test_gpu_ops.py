@@ -459,6 +459,30 @@ def test_matmul_split_products(gpu, bits, group, st, n_in, out, tokens):
         gpu.release(b_)
 
 
+@pytest.mark.parametrize("bits,n_in", [(2, 2048), (4, 2048), (8, 2048), (8, 4096)])
+def test_matmul_split_sum_of_groups(gpu, bits, n_in):
+    """The split products' running sum over groups of 32 rounds once per group:
+    within what an F32 sum of n_in / 32 terms of random sign rounds to (2^-24 /
+    sqrt(3) of it times sqrt(n / 2))."""
+    out, tokens = 300, 9
+    print(f"[case] split groups {bits}/32 [{n_in},{out}]", flush=True)
+    q = synth.quantize_affine(synth.normal(51 + bits, n_in * out, 0.0, 0.02), bits, 32, BF16)
+    t = Tensor.affine([n_in, out], *q, bits, 32, BF16)
+    x = synth.normal(52 + n_in, tokens * n_in).reshape(tokens, n_in)
+    w, xb, y = gpu.weight_tensor(t), gpu.upload(x), gpu.zeros(tokens * out)
+    with gpu.batch() as b:
+        b.matmul(w, xb, y, tokens)
+    # the weights as they are, code * scale + bias unrounded
+    codes = (q[0].reshape(-1, 1) >> np.arange(0, 32, bits, dtype=np.uint32)) & ((1 << bits) - 1)
+    s, c = (synth.bf16_bits_to_f32(v).astype(np.float64)[:, None] for v in q[1:])
+    wd = (codes.reshape(-1, 32) * s + c).reshape(out, n_in)
+    ref = x.astype(np.float64) @ wd.T
+    err = np.linalg.norm(gpu.read(y).reshape(tokens, out) - ref) / np.linalg.norm(ref)
+    assert err <= 2.0 ** -24 / np.sqrt(3) * np.sqrt(n_in / 32 / 2), err
+    for b_ in (xb, y):
+        gpu.release(b_)
+
+
 def test_matmul_split_nonfinite_rows(gpu):
     """A NaN or an infinity in a token's row reaches every output of that token
     and of no other."""
@@ -483,7 +507,7 @@ def test_matmul_split_infinities_and_overflow(gpu, bits, group, st, tokens):
     """Tiled products of rows the split has no finite value for: every output
     is the one its decoded weights give (oracle.matmul) -- an infinity of the
     products' sign, NaN where two meet or a weight is 0 -- and finite inputs of
-    about 2^121, whose sums overflow before the group's scale, give finite results."""
+    about 2^121 give finite results."""
     print(f"[case] split infinities {bits}/{group}/{st} tokens={tokens}", flush=True)
     n_in, out = 384, 70
     q = synth.quantize_affine(synth.normal(41 + bits, n_in * out, 0.0, 2.0 ** -8), bits, group, st)
