@@ -117,10 +117,9 @@ __device__ __forceinline__ void decode_w(const WRaw<BITS, T> &o, int j, float *v
 
 // CH: independent sums the products of a tile's K range go to in turn, added
 // pairwise at the end.  A single sum rounds once per product, so its error
-// grows with the range; dense rows of the batched router take eight over ranges
-// of at most 256 values (f32mm_ranges), which the wave sums of the VALU rows
-// match (two waves per SIMD, which their registers would just miss, are what the
-// grid fills).
+// grows with the range; the batched path's router takes eight over ranges of at
+// most 256 values (f32mm_ranges), which the wave sums of the VALU rows match (two
+// waves per SIMD, which their registers would just miss, are what the grid fills).
 template <int BITS, int T, bool GATE, int CH>
 __global__ __launch_bounds__(kThreads, CH == 8 ? 2 : 1) void f32mm_kernel(WDesc r, const float *__restrict__ x,
                                                               uint32_t tokens, uint32_t ksplit,
@@ -278,9 +277,7 @@ struct Launch {
     template <int BITS, int T>
     hipError_t operator()() {
         if (grow) return go<BITS, T, true, 1>();
-        if constexpr (BITS == 0)
-            if (chains == 8) return go<BITS, T, false, 8>();
-        return go<BITS, T, false, 1>();
+        return chains == 8 ? go<BITS, T, false, 8>() : go<BITS, T, false, 1>();
     }
     template <int BITS, int T, bool GATE, int CH>
     hipError_t go() {
@@ -318,9 +315,8 @@ uint32_t f32mm_ksplit(const WDesc &r, uint32_t tokens, uint64_t part_floats) {
 
 // K ranges of the batched path's router: no longer than 256 values, so that its
 // logits are no further from the 64-bit ones than those of the VALU rows it
-// replaces (h 2048, 512 rows: dense 1.23e-7 on VALU, here in one sum over 256
-// values 2.9e-7, in eight 1.23e-7; affine 3.2e-7 on VALU with uncentred codes,
-// here 2.9e-7).  0: their partial sums do not fit.
+// replaces (h 2048, 512 dense rows: 1.23e-7 on VALU, here in one sum over 256
+// values 2.9e-7, in eight 1.23e-7).  0: their partial sums do not fit.
 uint32_t f32mm_ranges(const WDesc &r, uint32_t tokens, uint64_t part_floats) {
     uint32_t ks = f32mm_ksplit(r, tokens, part_floats);
     if (r.in / ks > 256) ks = r.in % 256 == 0 ? r.in / 256 : r.in / 128;

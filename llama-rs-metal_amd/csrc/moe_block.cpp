@@ -314,19 +314,26 @@ moe_status run_batched(moe_gpu *g, const moe_block_weights *w, const Dims &d, co
     SideFork side{g, s};
     if (w->has_shared) TRY(side.mark());
     // The router's product stays F32 (no split: the routing is exact given the
-    // logits, so they are the F32 product's).  A router of many logits: the F32
-    // matrix cores (K split over the grid, its partial sums in y16, which this
-    // path leaves idle), from 2^15 logits on: 512 dense rows at 64 / 500 tokens
-    // 12 / 22 us against 32 / 239 on VALU.  Fewer: VALU rows, or, for affine rows
-    // they do not take (no 2^k chunks), the per-token wave (1024 -> 256 4-bit
-    // rows at 2 / 33 tokens 3.7 / 4.6 us, on the F32 matrix cores 26)
+    // logits, so they are the F32 product's): the F32 matrix cores (K split over
+    // the grid, its partial sums in y16, which this path leaves idle) from 12288
+    // logits and 16 tokens (affine: 56) on, VALU rows below.  A block of h 2048
+    // with its router on VALU / the matrix cores, us: dense, 512 experts at 12 /
+    // 16 / 24 / 63 tokens 90.4 / 93.0, 104.8 / 103.3, 135 / 128, 238 / 222, 128
+    // experts at 64 / 96 / 255 135.9 / 136.1, 149.6 / 145.8, 219 / 195; 4-bit, 512
+    // experts at 24 / 48 / 56 / 128 123 / 126, 186.7 / 187.5, 205.6 / 203.5, 304 /
+    // 286, 128 experts at 64 / 96 / 255 132.8 / 133.2, 145.8 / 144.5, 198 / 184;
+    // 1024 experts at 8 / 16 tokens dense 74 / 84, 111 / 108.
+    // Affine rows that VALU does not take (no 2^k chunks) and fewer logits: the
+    // per-token wave (h 640, 128 experts at 32 / 64 / 128 / 200 tokens 54.2 / 59.7
+    // / 69.8 / 79.7, on the matrix cores 59.8 / 63.3 / 69.0 / 73.3).
     const WDesc R = wdesc(w->router);
     uint32_t rks = 0;
-    if ((uint64_t)t32 * E >= (1u << 15) && f32mm_supported(R, xin)) rks = f32mm_ranges(R, t32, (uint64_t)T * K * d.h / 2);
+    if (T * E >= 12288u && t32 >= (R.bits ? 56u : 16u) && f32mm_supported(R, xin))
+        rks = f32mm_ranges(R, t32, (uint64_t)T * K * d.h / 2);
     float *parts = ws + L.y16;
     if (rks)
         TRY(launch_f32mm(p, s, "seg_router", R, xin, t32, rks, rks > 1 ? nullptr : bias, rks > 1 ? parts : logits,
-                         nullptr, nullptr, nullptr, R.bits ? 1 : 8));
+                         nullptr, nullptr, nullptr, 8));
     else if (seg_supported(R))
         TRY(launch_seg_rows(p, s, "seg_router", R, xin, nullptr, nullptr, nullptr, t32, seg_max_entries(t32, 0), bias,
                             logits));

@@ -93,8 +93,8 @@ hipError_t launch_route_sum(Prof *p, hipStream_t s, const float *parts, uint32_t
 // router's).  Profiled under `name`.
 bool f32mm_supported(const WDesc &w, const float *x);
 uint32_t f32mm_ksplit(const WDesc &w, uint32_t tokens, uint64_t part_floats);
-// The K ranges of the batched path's router (0: their partial sums do not fit);
-// dense rows are to be launched with eight `chains` (independent sums).
+// The K ranges of the batched path's router, launched with eight `chains`
+// (independent sums); 0: their partial sums do not fit.
 uint32_t f32mm_ranges(const WDesc &w, uint32_t tokens, uint64_t part_floats);
 // xb16 (optional, [tokens, in]): x rounded to bf16, written on the way.
 // grow: a dense F32 row (16-byte aligned) whose product with every token's x

@@ -384,12 +384,12 @@ def outlier_router(h, E, seed):
     return Tensor.affine([h, E], words.ravel(), s, b, 4, 64, BF16), cols
 
 
-@pytest.mark.parametrize("E,T", [(48, 100), (48, 190), (128, 200)])
+@pytest.mark.parametrize("E,T", [(48, 100), (48, 190), (128, 90), (128, 200)])
 def test_batched_affine_router_is_f32(gpu, E, T):
     """The batched path's affine router over inputs with a value of 2^30 in
     every 128, at weights of exactly 0: F32 products do not see it, f16 terms
-    scaled to it would keep 10 bits of the other inputs.  Few enough logits for
-    the VALU rows, 96 tokens and more."""
+    scaled to it would keep 10 bits of the other inputs.  On the VALU rows, and
+    from 12288 logits on the F32 matrix cores."""
     print(f"[case] affine router E={E} T={T}", flush=True)
     h = 256
     kinds = {"router": DENSE, "experts": (4, 64, BF16)}
@@ -402,22 +402,26 @@ def test_batched_affine_router_is_f32(gpu, E, T):
     assert rel_max_err(got[1], oracle.matmul(blk.router, x, T).reshape(T, E)) < 2e-6
 
 
-@pytest.mark.parametrize("h,T,kind", [(640, 2, (8, 64, BF16)), (640, 100, (4, 32, F32)), (384, 33, (2, 128, F16))])
+@pytest.mark.parametrize("h,T,kind", [(640, 2, (8, 64, BF16)), (640, 100, (4, 32, F32)), (384, 33, (2, 128, F16)),
+                                      (640, 260, (4, 64, BF16))])
 def test_batched_router_of_odd_rows_is_f32(gpu, h, T, kind):
     """An affine router whose rows the VALU lanes do not take (h no 2^k
-    chunks): the per-token F32 wave, with the logit bias added."""
+    chunks): the per-token F32 wave, with the logit bias added, and from 12288
+    logits the F32 matrix cores over ranges of 128 values."""
     print(f"[case] odd router h={h} T={T} kind={kind}", flush=True)
     kinds = {"router": kind, "experts": (4, 64, BF16)}
-    blk = HostBlock(h, 48, 4, 128, 0, kinds, seed=97 + T, random_experts=True)
+    E = 48 if T < 200 else 80
+    blk = HostBlock(h, E, 4, 128, 0, kinds, seed=97 + T, random_experts=True)
     x = synth.normal(4950 + T, T * h).reshape(T, h)
-    bias = hot_bias(T, 48, seed=T, frac=0.5, hot=5, boost=4.0)
+    bias = hot_bias(T, E, seed=T, frac=0.5, hot=5, boost=4.0)
     got, prof = profiled(gpu, lambda: run_block(gpu, blk.upload(gpu), x, T, PATH_AUTO, bias=bias))
-    assert "gemv_generic" in prof and "seg_gateup" in prof and "seg_router" not in prof, sorted(prof)
+    assert "seg_gateup" in prof and ("gemv_generic" in prof) != ("seg_router" in prof), sorted(prof)
+    assert ("seg_router" in prof) == (T * E >= 12288), sorted(prof)
     check_all_ids(blk, got)
     check_against_oracle(blk, x, got, bias=bias)
 
 
-@pytest.mark.parametrize("kind,T", [((4, 64, BF16), 128), ((8, 64, BF16), 128), (DENSE, 128), ((4, 64, BF16), 255)])
+@pytest.mark.parametrize("kind,T", [((4, 64, BF16), 90), ((4, 64, BF16), 128), ((8, 64, BF16), 128), (DENSE, 128), ((4, 64, BF16), 255)])
 def test_batched_routing_matches_oracle_f32_logits(gpu, kind, T):
     """The batched path's ids against the oracle's routing of its own F32
     logits: equal for every token whose K-th and K+1-th logits are further
@@ -451,6 +455,25 @@ def test_batched_dense_router_sums(gpu, kind, K, T):
     ref = x.astype(np.float64) @ np.asarray(oracle.decode(blk.router), np.float64).reshape(E, h).T
     err = np.linalg.norm(got[1] - ref) / np.linalg.norm(ref)
     assert err <= 2.0 ** -24 / np.sqrt(3) * np.sqrt(32 / 2), err
+
+
+@pytest.mark.parametrize("kind,E,T", [(DENSE, 800, 15), (DENSE, 800, 16), (DENSE, 128, 95), (DENSE, 128, 96),
+                                      ((4, 64, BF16), 256, 55), ((4, 64, BF16), 256, 56), ((8, 32, F32), 128, 95),
+                                      ((8, 32, F32), 128, 96), ((2, 128, F16), 200, 62)])
+def test_batched_router_on_both_sides(gpu, kind, E, T):
+    """The batched path's router on both sides of the lines between VALU rows
+    (routing and dispatch in one launch) and the F32 matrix cores (partial
+    sums): logits, ids and outputs against the oracle, with the logit bias."""
+    print(f"[case] router {kind} E={E} T={T}", flush=True)
+    h = 512
+    blk = HostBlock(h, E, 8, 128, 0, {"router": kind, "experts": (4, 64, BF16)}, seed=E + T, random_experts=True)
+    x = synth.normal(4995 + T, T * h).reshape(T, h)
+    bias = hot_bias(T, E, seed=T, frac=0.5, hot=6, boost=4.0)
+    got, prof = profiled(gpu, lambda: run_block(gpu, blk.upload(gpu), x, T, PATH_AUTO, bias=bias))
+    mfma = T * E >= 12288 and T >= (16 if kind == DENSE else 56)
+    assert ("route" in prof) == mfma and ("route_dispatch" in prof) == (not mfma), sorted(prof)
+    check_all_ids(blk, got)
+    check_against_oracle(blk, x, got, bias=bias)
 
 
 def test_more_runs_than_a_grid_holds(gpu):
