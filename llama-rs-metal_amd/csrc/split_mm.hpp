@@ -10,10 +10,12 @@
 // Why it is exact enough: an affine weight is code * scale + bias with a code
 // of at most 8 bits, and code - 2^(bits-1) is exact in f16.  An input value,
 // scaled by a power of two per row and 128 values, is split into two f16
-// terms hi + lo (hi rounded to nearest, lo the rounded remainder): 22 bits,
-// 2^-24 of it off on average.  So sum(code * x) over a quantization group is
-// two matrix products whose products are exact in the F32 accumulator, and the
-// group's scale and bias are applied to that sum in F32:
+// terms hi + lo (hi rounded to nearest, lo the rounded remainder): off by at
+// most 2^-22 of it (2^-24 on average), or, where that is smaller than lo's
+// subnormal spacing, by 2^-39 of the largest of the 128.  So sum(code * x) over
+// a quantization group is two matrix products whose single products are exact
+// (their sum rounds in the F32 accumulator), and the group's scale and bias are
+// applied to that sum in F32:
 //   out = sum_g scale_g * D_g + (bias_g + 2^(bits-1) scale_g) * sum_g(x),
 // a group's two terms first, so that the running sum rounds once per group.
 // The centred codes and the one F32 addition per group leave it closer to the

@@ -352,10 +352,10 @@ def test_batched_decode_layouts(gpu, experts, T):
 def test_batched_split_products(gpu, experts, ff, ffs, T):
     """The batched decode where the expert segments are long enough for the
     split products (and, with ff 384 and 640, where the VALU rows do not take the
-    down rows at any length, from one token on): ragged segments of 0 to over 32 pairs, segments that
-    end inside and at a 16-pair entry, the shared expert on either side of its
-    own threshold, every code width; and the router's F32 matrix-core product
-    where it has enough logits."""
+    down rows at any length, from one token on): ragged segments of 0 to 30
+    pairs, segments that end inside and at a 16-pair entry, the shared expert on
+    either side of its own threshold, every code width; and the router's F32
+    matrix-core product where it has enough logits."""
     print(f"[case] batched split experts={experts} ff={ff} ffs={ffs} T={T}", flush=True)
     E = 48 if T < 100 else 400
     kinds = {"router": (8, 64, BF16), "experts": experts, "shared": (4, 64, BF16), "shared_gate": DENSE}
@@ -368,6 +368,41 @@ def test_batched_split_products(gpu, experts, ff, ffs, T):
     check_all_ids(blk, got)
     check_against_oracle(blk, x, got, bias=bias)
     check_in_block_dispatch(bw, T, got[2], wsd["ws"], tm=bw.workspace_layout(T)["tile_pairs_batched"])
+
+
+@pytest.mark.parametrize("experts", [(2, 64, F16), (2, 128, BF16), (4, 32, F16), (4, 128, BF16), (8, 64, F32),
+                                     (8, 32, BF16)])
+@pytest.mark.parametrize("h,ff", [(640, 128), (1152, 384), (2048, 640)])
+def test_batched_split_long_rows(gpu, experts, h, ff):
+    """Split gate/up and down over rows of 5, 9 and 16 units (the scales'
+    reload every four, with and without a remainder), segments of 10 pairs on
+    average and of 40: three 16-pair entries, the last ragged.  h 640 and 1152
+    and ff 384 and 640 are split at any length.  F32 sums of 2048 products by
+    any two orders: within 1e-5 of the largest output."""
+    print(f"[case] batched split rows experts={experts} h={h} ff={ff}", flush=True)
+    T, E, K = 40, 16, 4
+    kinds = {"router": DENSE if h == 2048 else (8, 64, BF16), "experts": experts}
+    blk = HostBlock(h, E, K, ff, 0, kinds, seed=64 + h, random_experts=True)
+    x = synth.normal(4660 + h, T * h).reshape(T, h)
+    bias = hot_bias(T, E, seed=h, frac=1.0, hot=2, boost=30.0)
+    got = run_block(gpu, blk.upload(gpu), x, T, PATH_AUTO, bias=bias)
+    assert np.bincount(got[2].ravel(), minlength=E).max() == T
+    check_all_ids(blk, got)
+    check_against_oracle(blk, x, got, bias=bias, tol=1e-5)
+
+
+@pytest.mark.parametrize("bits,group,T", [(4, 64, 15), (4, 64, 16), (8, 64, 7), (8, 64, 8), (2, 32, 16), (4, 64, 95),
+                                          (4, 64, 96)])
+def test_batched_products_on_both_sides(gpu, bits, group, T):
+    """Both sides of the lines between VALU rows and split products: 1.5 pairs
+    an expert (0.75 at 8 bits), and 96 rows of the shared expert."""
+    print(f"[case] batched lines {bits}/{group} T={T}", flush=True)
+    kinds = {"router": DENSE, "experts": (bits, group, BF16), "shared": (bits, group, BF16), "shared_gate": DENSE}
+    blk = HostBlock(512, 64, 6, 128, 256, kinds, seed=66 + T, random_experts=True)
+    x = synth.normal(4670 + T, T * 512).reshape(T, 512)
+    got = run_block(gpu, blk.upload(gpu), x, T, PATH_AUTO)
+    check_all_ids(blk, got)
+    check_against_oracle(blk, x, got, tol=1e-5)
 
 
 def outlier_router(h, E, seed):

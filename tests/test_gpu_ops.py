@@ -438,7 +438,7 @@ def test_matmul_split_products(gpu, bits, group, st, n_in, out, tokens):
     """Batch::matmul of affine weights from 4 tokens on (split f16 products) at
     the edges of its tiles: one to nine units of 128 values, output rows and
     tokens around 16, both tile counts per wave, over rows of unlike magnitude
-    (2^-30 .. 2^30, one of zeros).  The bound per output is that of the method:
+    (2^-30 .. 2^30 from row to row, one of zeros).  The bound per output is that of the method:
     2^-22 of each product (the split of x) and F32 additions of one sum per
     group, under 2^-20 * sum |w x| together."""
     print(f"[case] split {bits}/{group}/{st} [{n_in},{out}] tokens={tokens}", flush=True)
@@ -479,6 +479,38 @@ def test_matmul_split_sum_of_groups(gpu, bits, n_in):
     ref = x.astype(np.float64) @ wd.T
     err = np.linalg.norm(gpu.read(y).reshape(tokens, out) - ref) / np.linalg.norm(ref)
     assert err <= 2.0 ** -24 / np.sqrt(3) * np.sqrt(n_in / 32 / 2), err
+    for b_ in (xb, y):
+        gpu.release(b_)
+
+
+@pytest.mark.parametrize("n_in,out,tokens", [(256, 40, 5), (1152, 130, 40)])
+def test_matmul_split_wide_units(gpu, n_in, out, tokens):
+    """Magnitudes of 2^-40 .. 2^0 and one of 2^30 inside every 128 values, the
+    largest at weights of exactly 0 (code 8 under scale s and bias -8 s), where
+    an F32 product would not see them.  The split is off by at most 2^-22 of a
+    value or 2^-39 of the largest of its 128, and the sums of the rest by F32's."""
+    print(f"[case] split wide units [{n_in},{out}] tokens={tokens}", flush=True)
+    rng = np.random.default_rng(n_in)
+    codes = rng.integers(0, 16, (out, n_in)).astype(np.uint32)
+    cols = np.arange(77, n_in, 128)
+    codes[:, cols] = 8
+    words = (codes.reshape(out, n_in // 8, 8) << (4 * np.arange(8, dtype=np.uint32))).sum(2, dtype=np.uint32)
+    n = out * n_in // 64
+    s = synth.f32_to_bf16_bits(np.full(n, 2.0 ** -7, np.float32))
+    b = synth.f32_to_bf16_bits(np.full(n, -(2.0 ** -4), np.float32))
+    t = Tensor.affine([n_in, out], words.ravel(), s, b, 4, 64, BF16)
+    x = synth.normal(53 + n_in, tokens * n_in).reshape(tokens, n_in)
+    x = (x * np.exp2(rng.integers(-40, 1, x.shape))).astype(np.float32)
+    x[:, cols] = np.float32(2.0 ** 30)
+    w, xb, y = gpu.weight_tensor(t), gpu.upload(x), gpu.zeros(tokens * out)
+    with gpu.batch() as bt:
+        bt.matmul(w, xb, y, tokens)
+    got = gpu.read(y).reshape(tokens, out).astype(np.float64)
+    wd = ((codes.astype(np.float64) - 8) * 2.0 ** -7)
+    x64 = x.astype(np.float64)
+    split = np.maximum(2.0 ** -22 * np.abs(x64), 2.0 ** -39 * 2.0 ** 30)
+    bound = split @ np.abs(wd).T + 2.0 ** -20 * (np.abs(x64) @ np.abs(wd).T)
+    assert np.all(np.abs(got - x64 @ wd.T) <= bound)
     for b_ in (xb, y):
         gpu.release(b_)
 
