@@ -1,5 +1,6 @@
-// Batched decode: T >= 2 tokens whose expert segments are too short for the
-// bf16 MFMA path (config 3: 8 to 64 tokens over 512 experts).  The fused
+// Batched decode: tokens whose expert segments are too short for the bf16 MFMA
+// path (config 3: 8 to 64 tokens over 512 experts), and single tokens of layers
+// the fused decode does not take.  The fused
 // decode's lane layout (lanerows.hpp) runs over work entries of at most
 // kSegTokens rows of input: a wave loads its weight rows once and applies
 // them to every input row of its entry, so every expert row is read from HBM
@@ -11,9 +12,10 @@
 //               expert over all tokens -> act [pair or token, ff]
 //   seg_rows    plain row products of input row p -> out[p, row]: the router
 //               (Batch::matmul(router), execute.rs:220, with the logit bias
-//               added), the routed down rows (expert_matmul(down),
-//               execute.rs:225), the shared expert's down rows and its gate
-//               input row (execute.rs:228-230)
+//               added) below 12288 logits, the routed down rows
+//               (expert_matmul(down), execute.rs:225) and the shared expert's
+//               (execute.rs:228-230)
+// Longer segments and rows of no 2^k chunks are split products (k_split.hip).
 //
 // Entries: either the dispatch's segments cut into runs of kSegTokens pairs
 // (tile_schedule: (expert, first pair); the run ends at the segment end), or

@@ -437,7 +437,8 @@ static bool pow2_chunks(uint32_t n) {
     return c >= 1 && c <= 64 && (c & (c - 1)) == 0;
 }
 // Rows of ff values: 2^k or 3 * 2^k chunks of 32, at most 64 lanes of one or
-// three chunks (0: neither; those layers take the grouped path).  With three
+// three chunks (0: neither; those layers take the batched path where the split
+// products do, whole units of 128 values, else the grouped one).  With three
 // chunks a lane the 128-expert layer of ff 768 decodes in 18.3 us (decode_down
 // 4.7), against 104 on the grouped path, whose wave walks one row at a time
 // with a load per word in flight.

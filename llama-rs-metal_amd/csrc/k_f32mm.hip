@@ -1,14 +1,16 @@
 // F32 products on the F32 matrix cores (v_mfma_f32_32x32x2_f32):
 // y[t, r] = x_t . W_r (+ bias), W dims [in, out] (dense F32/F16/BF16 or
 // affine 2/4/8-bit).  Two callers:
-//  - the router product of the prefill path, Batch::matmul(router)
+//  - the router product of the prefill path, and of the batched path from
+//    12288 logits on, Batch::matmul(router)
 //    (crates/model-runtime/src/execute.rs:220).  The routing is exact given
 //    the logits, so the logits themselves must be F32 products: bf16
 //    operands change the selected experts of about 1-2% of the tokens of a
 //    4096-token prefill;
 //  - moe_matmul at 4 tokens or more, where the reference switches from its
 //    GEMV kernels to tiled F32 GEMMs (affine_mm, gemm_simd / gemm_simd_wide,
-//    crates/metal-backend/src/apple/ops/matrix.rs:77-123).
+//    crates/metal-backend/src/apple/ops/matrix.rs:77-123): dense weights, and
+//    affine ones that the split products (k_split.hip) do not take.
 // Both operands stay F32: x as given, and the weights decoded to F32 exactly
 // as Tensor::decode does (w = code * scale + bias, one product and one sum,
 // crates/model-format/src/checkpoint.rs:164-196; F16/BF16 widened exactly).

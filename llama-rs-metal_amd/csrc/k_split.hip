@@ -25,12 +25,20 @@ static hipError_t split_dispatch(const split::Launch &l, int mode) {
 // Where the split products overtake the VALU rows of k_batched.hip, which cost
 // about one instruction per code and input row against a fixed cost per code:
 //  - over dispatched segments, from 1.5 pairs an expert on average (0.75 at 8
-//    bits, whose conversions the VALU rows repeat per input).  Gate/up + down of
-//    512 experts of h 2048, ff 512 at 64 / 100 / 300 tokens (1.25 / 2 / 5.9
-//    pairs): 4-bit 183 / 254 / 623 us on VALU, 201 / 239 / 286 split; 2-bit 207
-//    / 294 against 223 / 257; 8-bit at 16 / 64: 105 / 299 against 112 / 258;
+//    bits, whose conversions the VALU rows repeat per input), amid the crossings
+//    of three layers of h 2048.  A layer on VALU / split, us, at these pairs:
+//      512 experts, ff 512: 2-bit 1.25 253 / 262, 1.5 291 / 278; 4-bit 1.25 232 /
+//        242, 1.5 260 / 262, 1.75 285 / 273; 8-bit 0.47 185 / 187, 0.62 226 / 216
+//      128 experts, ff 512: 2-bit 1.25 85.6 / 85.0, 1.5 95 / 97, 1.75 106 / 97;
+//        4-bit 1.25 83 / 80, 1.5 88 / 90, 1.75 94 / 90; 8-bit (group 64) 0.5 71.5
+//        / 73.2, 0.75 81.7 / 85.0, 1 94.8 / 93.4
+//      128 experts, ff 768: 2-bit 1.5 117 / 120, 2 130 / 131, 2.5 149 / 138; 4-bit
+//        1.25 101 / 105, 1.5 114 / 112; 8-bit 0.5 85.7 / 85.6, 0.75 108 / 107;
 //  - over all tokens, from 96 rows: the shared expert's three products at 64 /
-//    100 / 300 tokens 23 / 35 / 82 us against 25 / 26 / 38.
+//    100 / 300 tokens 23 / 35 / 82 us against 25 / 26 / 38 on their own.
+// Rows VALU does not take are split at any count (the grouped path instead: ff
+// 640 at 1 / 2 / 8 tokens of 128 experts 73 / 115 / 209 us a layer, split 32 / 37
+// / 64).
 bool split_rows_better(const WDesc &w, uint32_t n, uint32_t experts) {
     if (experts <= 1) return n >= 96;
     return w.bits == 8 ? 4ull * n >= 3ull * experts : 2ull * n >= 3ull * experts;
@@ -65,7 +73,8 @@ hipError_t launch_split_rows(Prof *p, hipStream_t s, const char *name, const WDe
     const uint64_t blocks1 = (uint64_t)((w.out + 63) / 64) * ((n + split::kRows - 1) / split::kRows);
     const int nt = !tiles && blocks1 <= 512 ? 1 : 2;
     // grid.y is limited to 65535 entries: longer runs of input rows in parts
-    // (dispatched segments are at most 65535 tokens' pairs, and far fewer runs)
+    // (dispatched segments come with at most 65535 runs: block_entry sends more
+    // to the grouped path)
     const uint32_t part = tiles ? n : 65535u * split::kRows;
     hipError_t e = hipSuccess;
     for (uint64_t n0 = 0; n0 < n && e == hipSuccess; n0 += part) {

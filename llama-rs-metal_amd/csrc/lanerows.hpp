@@ -59,11 +59,13 @@ struct Chunk32 {
     // (code - kCentre), so that the sum and its rounding stay small.  rs: the
     // sums of x over its runs of kRun (run_sums; affine rows only).
     // F16 = false: each run's chain of FMAs over the unsigned codes starts at
-    // -kCentre times the run's sum (shorter runs at 8 bits, whose centre is the
-    // larger against what the sum comes to).  The shortest code (4-byte
-    // conversions and FMAs), for waves that run through their rows once:
-    // decode_gateup 7.7 us against 8.5 with F16.
-    // F16 = true: eight codes at a time to centred f16 (codes16.hpp),
+    // -kCentre times the run's sum.  The shortest code (4-byte conversions and
+    // FMAs), for waves that run through their rows once: decode_gateup 7.7 us
+    // against 8.5 with F16.  Runs of four: a 4-bit decode layer of 512 / 128
+    // experts is 3.2e-7 / 3.2e-7 off its 64-bit result in 17.05 / 16.1 us, with
+    // runs of eight 3.8e-7 / 4.1e-7 in 16.85 / 15.9 (8-bit, 512 experts, 3.0e-7
+    // in 19.4 us; over uncentred codes 7.5e-7 in 19.05).
+    // F16 = true (4 bits): eight codes at a time to centred f16 (codes16.hpp),
     // multiplied by mixed-precision FMAs: fewer instructions, for waves whose
     // arithmetic repeats over inputs (seg_down at 64 tokens 90 -> 68 us).
     static constexpr int kRun = BITS == 2 ? 8 : 4;
@@ -71,15 +73,14 @@ struct Chunk32 {
     template <bool F16>
     __device__ __forceinline__ float dot(const float *x, [[maybe_unused]] const float *rs) const {
         float d = 0.f;
-        if constexpr (BITS && F16) {
+        static_assert(!F16 || BITS == 4, "f16 conversion takes 4-bit codes");
+        if constexpr (F16) {
             codes16::Magic mg;
             mg.pin();
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 // codes (0, 4), (1, 5), (2, 6), (3, 7) of the run
-                const codes16::f16x8 c = BITS == 2   ? codes16::code_frag<BITS>(w[i >> 1], 0, i & 1, mg)
-                                         : BITS == 4 ? codes16::code_frag<BITS>(w[i], 0, 0, mg)
-                                                     : codes16::code_frag<BITS>(w[2 * i], w[2 * i + 1], 0, mg);
+                const codes16::f16x8 c = codes16::code_frag<4>(w[i], 0, 0, mg);
                 float r = 0.f;
 #pragma unroll
                 for (int j = 0; j < 8; j++) r = fmaf((float)c[j], x[8 * i + (j >> 1) + 4 * (j & 1)], r);

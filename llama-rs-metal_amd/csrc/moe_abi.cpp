@@ -305,7 +305,9 @@ moe_status moe_matmul(moe_gpu *g, const moe_weight *w, moe_buffer x, moe_buffer 
     // affine_mm / gemm_simd (matrix.rs:77-123); fewer: one GEMV per token.
     // Affine weights as split products on the f16 matrix cores (h 2048 -> 4096
     // 4-bit rows at 4 / 256 / 2000 tokens 12 / 26 / 144 us, on the F32 matrix
-    // cores 47 / 52 / 280, and a fifth of their error), the rest on the F32 ones
+    // cores 47 / 52 / 280; 512 -> 2048, 2048 -> 512, 4096 -> 1000 and 1024 -> 256
+    // at 2, 4 and 8 bits and 4 to 500 tokens 0.2 to 0.7 of those; a fifth of
+    // their error), the rest on the F32 ones
     if (tokens >= 4 && split_supported(d, (const float *)x.ptr))
         return launched(g, launch_split_rows(&g->prof, g->stream, "matmul_f32", d, (const float *)x.ptr, nullptr,
                                              nullptr, nullptr, (uint32_t)tokens, 0, (float *)y.ptr),
