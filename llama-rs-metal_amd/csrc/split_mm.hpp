@@ -388,7 +388,7 @@ __device__ __forceinline__ void body(const Args &a, Stage *st, uint32_t bx, uint
                 const float s = Scales<T, GS>::value(sw[t][0], g);
                 const float b = fmaf((float)(1 << (BITS - 1)), s, Scales<T, GS>::value(sw[t][1], g));
 #pragma unroll
-                for (int r = 0; r < 4; r++) acc[t][r] = fmaf(fmaf(b, xs[r], s * d[t][r]), fx[r], acc[t][r]);
+                for (int r = 0; r < 4; r++) acc[t][r] = fmaf(fmaf(s, d[t][r], b * xs[r]), fx[r], acc[t][r]);
                 // the group's sums are added here: left to itself the compiler
                 // sinks every group's additions below the last one's products,
                 // holding all their sums (half as many waves fit)
@@ -430,7 +430,7 @@ __device__ __forceinline__ void body(const Args &a, Stage *st, uint32_t bx, uint
         if (u + 3 < units) unit(u + 3, std::integral_constant<int, 3>{});
     }
     // acc[t][r]: input row 4 q + r, weight row 16 t + n16
-    uint32_t redo = 0;  // bit kOut * r + t: an output that is not finite
+    float bad = 0.f;  // NaN once an output is not finite
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const uint32_t p = beg + 4 * q + r;
@@ -441,20 +441,23 @@ __device__ __forceinline__ void body(const Args &a, Stage *st, uint32_t bx, uint
             if (c >= out) continue;
             float v = acc[t][r];
             if constexpr (MODE == GATEUP) v = v / (1.0f + expf(-v)) * acc[t + kOut][r];
-            if (!__builtin_isfinite(v)) redo |= 1u << (kOut * r + t);
+            bad = fmaf(v, 0.f, bad);
             a.out[(uint64_t)p * out + c] = v;
         }
     }
-    while (redo) {
-        const int i = __builtin_ctz(redo);
-        redo &= redo - 1;
+    if (bad == 0.f) return;
+#pragma unroll 1
+    for (int i = 0; i < 4 * kOut; i++) {
         const uint32_t p = beg + 4 * q + i / kOut, c = col0 + 16 * (i % kOut) + n16;
+        if (p >= end || c >= out) continue;
+        float &o = a.out[(uint64_t)p * out + c];
+        if (__builtin_isfinite(o)) continue;
         const uint64_t row = ((uint64_t)e * out + c) * in;
         const uint32_t src = MODE == GATEUP && a.perm ? a.perm[p] / a.k : p;
         const float *x = a.in + (uint64_t)src * in;
         float v = decoded_dot<BITS, T>(a.w, row, x);
         if constexpr (MODE == GATEUP) v = v / (1.0f + expf(-v)) * decoded_dot<BITS, T>(a.w2, row, x);
-        a.out[(uint64_t)p * out + c] = v;
+        o = v;
     }
 }
 
