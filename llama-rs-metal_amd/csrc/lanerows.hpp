@@ -62,9 +62,11 @@ struct Chunk32 {
     // -kCentre times the run's sum.  The shortest code (4-byte conversions and
     // FMAs), for waves that run through their rows once: decode_gateup 7.7 us
     // against 8.5 with F16.  Runs of four: a 4-bit decode layer of 512 / 128
-    // experts is 3.2e-7 / 3.2e-7 off its 64-bit result in 17.05 / 16.1 us, with
-    // runs of eight 3.8e-7 / 4.1e-7 in 16.85 / 15.9 (8-bit, 512 experts, 3.0e-7
-    // in 19.4 us; over uncentred codes 7.5e-7 in 19.05).
+    // experts without a norm is 3.2e-7 / 3.2e-7 off its 64-bit result in 17.05 /
+    // 16.1 us, with runs of eight 3.8e-7 / 4.1e-7 in 16.85 / 15.9, over uncentred
+    // codes 5.2e-7 in 16.9 (512 experts; with a norm 17.75 us all three).  8 bits,
+    // 512 experts: 3.0e-7 in 19.4 us (with a norm 20.2), uncentred 7.5e-7 in 19.05
+    // (20.3); as signed bytes 2.3e-7 in 19.0, but 20.5 with a norm.
     // F16 = true (4 bits): eight codes at a time to centred f16 (codes16.hpp),
     // multiplied by mixed-precision FMAs: fewer instructions, for waves whose
     // arithmetic repeats over inputs (seg_down at 64 tokens 90 -> 68 us).
