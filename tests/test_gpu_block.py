@@ -494,14 +494,17 @@ def test_batched_dense_router_sums(gpu, kind, K, T):
 
 @pytest.mark.parametrize("kind,E,T", [(DENSE, 800, 15), (DENSE, 800, 16), (DENSE, 128, 95), (DENSE, 128, 96),
                                       ((4, 64, BF16), 256, 55), ((4, 64, BF16), 256, 56), ((8, 32, F32), 128, 95),
-                                      ((8, 32, F32), 128, 96), ((2, 128, F16), 200, 62)])
+                                      ((8, 32, F32), 128, 96), ((2, 128, F16), 200, 62), (DENSE, 1100, 16),
+                                      ((4, 32, BF16), 1500, 60)])
 def test_batched_router_on_both_sides(gpu, kind, E, T):
     """The batched path's router on both sides of the lines between VALU rows
     (routing and dispatch in one launch) and the F32 matrix cores (partial
-    sums): logits, ids and outputs against the oracle, with the logit bias."""
+    sums), and past 1024 experts: logits, ids and outputs against the oracle,
+    with the logit bias."""
     print(f"[case] router {kind} E={E} T={T}", flush=True)
     h = 512
-    blk = HostBlock(h, E, 8, 128, 0, {"router": kind, "experts": (4, 64, BF16)}, seed=E + T, random_experts=True)
+    K = 8 if E <= 1024 else 12
+    blk = HostBlock(h, E, K, 128, 0, {"router": kind, "experts": (4, 64, BF16)}, seed=E + T, random_experts=True)
     x = synth.normal(4995 + T, T * h).reshape(T, h)
     bias = hot_bias(T, E, seed=T, frac=0.5, hot=6, boost=4.0)
     got, prof = profiled(gpu, lambda: run_block(gpu, blk.upload(gpu), x, T, PATH_AUTO, bias=bias))
