@@ -27,7 +27,8 @@ hipError_t launch_route(Prof *p, hipStream_t s, const float *logits, uint32_t ex
 }
 
 // Routing of router products split over K: logits[t, j] = sum_s part[s, t, j]
-// (s ascending) + bias[t, j], written out and routed by the token's wave.
+// (pairs of ranges first) + bias[t, j], written out and routed by the token's
+// wave.
 // Latency-bound: a token's partial sums are a few dozen KB read by one wave,
 // so kSumParts of them are in flight per lane at a time, four logits each
 // (VEC: E % 4 == 0 and 16-byte aligned arrays).  One load at a time took 35 us

@@ -86,7 +86,8 @@ hipError_t launch_route_sum(Prof *p, hipStream_t s, const float *parts, uint32_t
                             const float *bias, uint32_t experts, uint32_t k, int normalize,
                             uint32_t tokens, float *logits, uint32_t *ids, float *weights);
 // out[t, r] = x_t . W_r in F32 on the F32 matrix cores (k_f32mm.hip; the
-// prefill router product and moe_matmul at >= 4 tokens), W 2-D: K split
+// prefill and batched router products and moe_matmul of dense weights at >= 4
+// tokens), W 2-D: K split
 // into `ksplit` ranges (f32mm_ksplit picks it for a partial buffer of
 // `part_floats`); with ksplit 1 `out` receives the products (+ bias), else
 // the partial sums [ksplit, tokens, out] (launch_route_sum adds the
@@ -100,7 +101,8 @@ uint32_t f32mm_ranges(const WDesc &w, uint32_t tokens, uint64_t part_floats);
 // grow: a dense F32 row (16-byte aligned) whose product with every token's x
 // the router also forms, one partial sum per K range and column of 128
 // outputs: gout[(kr * f32mm_columns(w) + c) * tokens + t]; a K range
-// (w.in / ksplit) of at most f32mm_gate_max() values
+// (w.in / ksplit) of at most f32mm_gate_max() values.  chains: 1, or 8 (without
+// grow) for sums that round less.
 uint32_t f32mm_gate_max();
 uint32_t f32mm_columns(const WDesc &w);
 hipError_t launch_f32mm(Prof *p, hipStream_t s, const char *name, const WDesc &w, const float *x,
